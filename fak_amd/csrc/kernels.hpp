@@ -59,6 +59,11 @@ int q4k_gemm32(const void *W, const float *X, float *Y, int N, int K, int M);
 size_t gemm32_ws_bytes(int fmt, int N, int K, int M);
 // The same GEMM over a tiled Q6_K weight (prefill of the q4_k_m Q6_K tensors).
 int q6k_gemm32(const void *W, const float *X, float *Y, int N, int K, int M);
+// Y[i] = part[i] + part[total + i] + ... over SK ranges, in range order.
+int sum_ranges(const float *part, float *Y, int SK, int total);
+// More tokens of a tiled Q8_0 weight (q8_0_gemm.hip), at most kQ8GemmTokens per call.
+constexpr int kQ8GemmTokens = 1024;
+int q8_0_gemm(const void *W, const float *X, float *Y, int N, int K, int M);
 int q8_0_gemv(const void *W, const float *X, float *Y, int N, int K, int M);
 
 // __builtin_amdgcn_sched_barrier mask: every instruction class except vector-memory ones may be
@@ -92,6 +97,24 @@ __device__ __forceinline__ uint32_t ld_stream32(const void *p) {
 }
 __device__ __forceinline__ uint16_t ld_stream16(const void *p) {
   return __builtin_nontemporal_load(reinterpret_cast<const uint16_t *>(p));
+}
+
+// A direct-to-LDS load of 16 (4) bytes per lane from base + soff + voff (base and soff uniform) to
+// dst + 16 (4) * lane. A buffer load: the scalar resource and offset leave one lane offset register that
+// lives for the whole kernel, where a flat load needs its 64-bit addresses rebuilt per load.
+// The compiler tracks these loads per LDS object (at most eight): an LDS read whose object it knows
+// waits only for that object's loads, any other LDS read for every load in flight. It loses the
+// object when the read's address is built in several steps, so such reads index a named array with
+// one opaque register (in_reg).
+__device__ __forceinline__ void lds_load16(const void *base, void *dst, int voff, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, 0xFFFFFFFFu, 0x00020000),
+      (__attribute__((address_space(3))) void *)dst, 16, voff, soff, 0, 0);
+}
+__device__ __forceinline__ void lds_load4(const void *base, void *dst, int voff, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, 0xFFFFFFFFu, 0x00020000),
+      (__attribute__((address_space(3))) void *)dst, 4, voff, soff, 0, 0);
 }
 
 // v + p[0] + p[stride] + ... + p[(N - 1) stride], in that order, every load issued first.

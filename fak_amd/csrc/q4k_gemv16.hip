@@ -585,6 +585,18 @@ __global__ __launch_bounds__(64) void gemv16_reduce_wide_kernel(const float *__r
 
 }  // namespace
 
+int sum_ranges(const float *part, float *Y, int SK, int total) {
+  if (SK >= 8 && SK <= kRangesAtOnce)
+    gemv16_reduce_wide_kernel<<<ceil_div(total, 64), 64, 0, stream()>>>(part, Y, SK, total);
+  else if (total % 4 == 0 && ((uintptr_t)Y & 15) == 0)
+    gemv16_reduce_kernel<<<ceil_div(total / 4, 256), 256, 0, stream()>>>(
+        (const float4 *)part, (float4 *)Y, SK, total / 4);
+  else
+    gemv16_reduce1_kernel<<<ceil_div(total, 256), 256, 0, stream()>>>(part, Y, SK, total);
+  FHIP_CHECK_LAUNCH("gemv16_reduce_kernel");
+  return FHIP_OK;
+}
+
 // K ranges per call: ranges of 4 super-blocks when K allows it, else of 4 to 5 (the kernel
 // works in passes of two super-blocks, so an odd range pads one; measured at the 7B / 27B FFN
 // shapes at 16 tokens, longer ranges lose parallelism and shorter ones pay more per-range start
@@ -614,17 +626,7 @@ int launch_gemv16(const void *Wv, const float *X, float *Y, int N, int K, int M)
   quant_gemv16_kernel<FMT, T32><<<nrb * SK, 256, 0, stream()>>>((const uint8_t *)Wv, X, Y, part, N, K,
                                                             M, nblk, ntiles, SK);
   FHIP_CHECK_LAUNCH("quant_gemv16_kernel");
-  if (SK > 1) {
-    const int tot = M * N;
-    if (SK >= 8 && SK <= kRangesAtOnce)
-      gemv16_reduce_wide_kernel<<<ceil_div(tot, 64), 64, 0, stream()>>>(part, Y, SK, tot);
-    else if (tot % 4 == 0 && ((uintptr_t)Y & 15) == 0)
-      gemv16_reduce_kernel<<<ceil_div(tot / 4, 256), 256, 0, stream()>>>(
-          (const float4 *)part, (float4 *)Y, SK, tot / 4);
-    else
-      gemv16_reduce1_kernel<<<ceil_div(tot, 256), 256, 0, stream()>>>(part, Y, SK, tot);
-    FHIP_CHECK_LAUNCH("gemv16_reduce_kernel");
-  }
+  if (SK > 1) return sum_ranges(part, Y, SK, M * N);
   return FHIP_OK;
 }
 }  // namespace

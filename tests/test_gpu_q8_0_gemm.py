@@ -1,0 +1,48 @@
+"""The Q8_0 GEMM (q8_gemm_kernel) at the edges of its tiles: rows around the workgroup's 128, one
+block to an odd number of them, ranges shorter than its three-pair passes, 17 tokens (two where the
+operands do not fit in the GEMV's LDS) to more than a slice of 1024, against the weights dequantized on the host in 64 bits.
+
+Tolerance: an activation enters as two f16 operands, 22 bits below the largest magnitude of its
+range (4 to 5 RMS here), so an output's error is about 1e-6 RMS, and its f32 sums add a few 2^-24 per
+block: 1e-5 max|d|/RMS is several times both."""
+import numpy as np
+import pytest
+
+from fak_amd import synth
+from tests.gpu_util import q8_0_matmul, rel_err_rows, scaled_activations
+
+pytestmark = pytest.mark.gpu
+
+
+def exact(raw, out, in_, X):
+    blk = raw.reshape(out, in_ // 32, 34)
+    d = blk[:, :, 0:2].copy().view(np.float16).astype(np.float64)
+    w = (blk[:, :, 2:].view(np.int8).astype(np.float64) * d).reshape(out, in_)
+    return X.astype(np.float64) @ w.T
+
+
+@pytest.mark.parametrize("out,in_,P", [(1, 32, 17), (127, 64, 32), (129, 96, 33), (260, 544, 64),
+                                       (1536, 576, 65), (513, 3584, 200), (40, 18944, 96),
+                                       (3584, 1056, 128), (48, 1024, 1061), (2100, 4096, 150),
+                                       (16, 18944, 2), (300, 9216, 5), (65, 3584, 12)])
+def test_shapes(hip, out, in_, P):
+    print(f"[case] q8_0 gemm out={out} in={in_} P={P}", flush=True)
+    raw = synth.q8_0_weights(out, in_, seed=out + in_)
+    X = synth.activations(P, in_, P)
+    assert rel_err_rows(q8_0_matmul(raw, out, in_, X, P), exact(raw, out, in_, X)) <= 1e-5
+
+
+@pytest.mark.parametrize("pattern", ["all", "wee"])
+def test_scales_and_special_values(hip, pattern):
+    """Any finite activation scale, and a NaN or an infinity stays in its own token."""
+    out, in_, P = 200, 2048, 40
+    print(f"[case] q8_0 gemm {pattern}", flush=True)
+    raw = synth.q8_0_weights(out, in_, seed=3)
+    X = scaled_activations(P, in_, 5, pattern)
+    ref = exact(raw, out, in_, X)
+    X[7, 100], X[20, 2047] = np.nan, -np.inf
+    Y = q8_0_matmul(raw, out, in_, X, P)
+    assert np.isnan(Y[[7, 20]]).all()
+    keep = [t for t in range(P) if t not in (7, 20)]
+    # a row of one huge value is held to its RMS: 22 bits below it
+    assert rel_err_rows(Y[keep], ref[keep]) <= 1e-5
