@@ -88,7 +88,7 @@ struct W16<1> {
   uint2 q[2][2][3];  // [K half hh][lane group h][ql a, ql b, qh]
 };
 
-// T32 (17..32 tokens): the 32 operand rows are 32 tokens, each the f16 of x / s_t with no
+// T32 (17..32 tokens, Q6_K): the 32 operand rows are 32 tokens, each the f16 of x / s_t with no
 // remainder row (the prefill GEMM's activation precision), the Q4_K min term's rows S_s / 32 in
 // f16; one 32-row tile per wave (for Q4_K the second token's staging registers leave no room for
 // two; Q6_K always runs one).
@@ -645,13 +645,9 @@ int q6k_gemv16(const void *Wv, const float *X, float *Y, int N, int K, int M) {
   return launch_gemv16<1>(Wv, X, Y, N, K, M);
 }
 
-// 17..32 tokens of a Q4_K matmul, at the prefill GEMM's activation precision (f16 of x / s per
-// token and K range): a chunk of a few tens of tokens costs about what 16 do here, where the
-// 128-token tile of the prefill GEMM costs nearly what 128 do.
-int q4k_gemv32(const void *Wv, const float *X, float *Y, int N, int K, int M) {
-  return launch_gemv16<0, true>(Wv, X, Y, N, K, M);
-}
-
+// 17..32 tokens, at the prefill GEMM's activation precision (f16 of x / s per token and K range): a
+// chunk of a few tens of tokens costs about what 16 do here, where the 128-token tile of the prefill
+// GEMM costs nearly what 128 do. (Q4_K takes q4k_mid.hip.)
 int q6k_gemv32(const void *Wv, const float *X, float *Y, int N, int K, int M) {
   return launch_gemv16<1, true>(Wv, X, Y, N, K, M);
 }
