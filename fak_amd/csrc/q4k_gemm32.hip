@@ -17,7 +17,7 @@
 // as both operands use it: here the K16 slice q holds positions 16q + 8 (lane / 32) + perm8(j),
 // which is where the nibble unpack leaves the weights.
 //
-// Q4_K runs q4k_gemm32s_kernel<4>: the same tile and K order with four waves of 128 tokens x
+// The default is quant_gemm32s_kernel: the same tile and K order with four waves of 128 tokens x
 // 32 rows each and activations staged by direct-to-LDS loads (described there).
 //
 // The same kernel runs Q6_K weights (FMT 1) from the Q6_K tiled records (tiled.hpp): the K16
@@ -25,6 +25,8 @@
 // and one 16-byte qh unit (a 2-bit field); a lane takes the 8 codes of its half (8 kap ..) and
 // makes w = (c - 32) * f16(d * sc) in f16: (1024 + c) - 1056 is exact, one rounding for the
 // product.
+#include <type_traits>
+
 #include "kernels.hpp"
 
 namespace fhip {
@@ -499,38 +501,45 @@ constexpr int wait_vm(int n) { return 0x0070 | (n & 15) | ((n >> 4) << 14); }  /
 //   * each of the four waves owns all 128 tokens x 32 rows (4 MFMA tiles), so every dequantized
 //     weight operand feeds four MFMAs instead of two and each weight is dequantized once per
 //     workgroup (the four-wave 2x2 form dequantizes every row twice);
-//   * activations go global -> LDS directly (global_load_lds_dwordx4, no staging registers) in
-//     8 KB stages of two K16 slices {h, 2 + h} of a 64-K chunk, four stage buffers, each stage
-//     loaded three stages ahead; every load is issued unconditionally (indices clamped at the
-//     end of K) so each wait is a compile-time count that leaves the later stages in flight;
+//   * activations go global -> LDS directly (lds_load16, no staging registers) in 16 KB stages of a
+//     64-K chunk; every load is issued unconditionally (indices clamped at the end of K) so each wait
+//     is a compile-time count that leaves the later stages in flight. A chunk per stage, not half of
+//     one, halves the barriers and the address arithmetic: 512 / 2048 tokens of 18944 x 3584 85.5 /
+//     282 -> 82.6 / 276 us, of Q6_K 97.7 / 329 -> 94.0 / 317, 3584 x 18944 117.5 / 366 -> 114.5 / 357;
 //   * the weights go straight from the tiled records to the registers of the lanes that use
 //     them (a header and four nibble units per lane and super-block), with no LDS round trip and
 //     no second barrier per super-block (measured 4-5% faster than records staged through LDS
 //     at M = 128 / 512 / 2048: 41.5 / 97 / 367 us against 43.6 / 100-103 / 382-394).
-// 166 VGPRs and 33 KB of LDS: three workgroups (12 waves) per CU, so the 592 workgroups of
-// M=512 spread to at most three 32-row waves per SIMD. Two waves of 64 rows per workgroup
-// (256 VGPRs, two per SIMD) measured slower at every size (M=512 112.7 against 106.5 us, M=2048
-// 413 against 376, with the records still in LDS) and no longer fit their registers.
+// Three forms (plan_gemm32): 128-row workgroups with two stage buffers (33 KB of LDS, 163 VGPRs, three
+// workgroups per CU), each half of a super-block's records reloaded as its last use is read out; DEEP,
+// the same with four buffers (three stages ahead) and the next super-block's records all in flight
+// under the current one (198 VGPRs, two per CU); and 256-row workgroups with four buffers (two per
+// CU).
 constexpr int kGemmWaves = 4;
-// Loads a wave may leave pending at the end of stage ls (0..7) of a super-block, with nt 32-row
-// tiles per wave: the DMA of the two later stages (kdma each), and for Q6_K the record group
-// issued at stage 0 (6 nt loads) through stage 2 and the one issued at stage 4 (8 nt loads)
-// through stage 6. Q4_K's records (2 nt and 3 nt loads) complete within the stage after their
-// issue: with plain loads pending beside the LDS DMA the compiler no longer trusts the counter's
-// order and drains it (vmcnt(0)) before the next read of a DMA buffer, twice per super-block,
-// which measured the same.
-constexpr int gemm32s_wait(int fmt, int nt, int ls, int kdma) {
-  return fmt == 0 ? 2 * kdma + (ls <= 1 ? 2 * (nt - 1) : 0) + (ls == 4 || ls == 5 ? 3 * (nt - 1) : 0)
-                  : 2 * kdma + (ls <= 2 ? 6 * nt : 0) + (ls >= 4 && ls <= 6 ? 8 * nt : 0);
+// Loads a wave may leave pending at the end of chunk stage c (0..3) of a super-block: the DMA (4 loads)
+// of the stages after s + 1, and the record loads issued after stage s + 1's DMA. Records: with
+// kNoLoadAcross they stay behind their stage's DMA, at chunk 0 (u1: the second half's units; DEEP: all
+// of the next super-block's) and chunk 2 (hu0: the next super-block's header and first half).
+constexpr int kNoLoadAcross = 0x38F;  // everything but vector memory
+constexpr int gemm32s_wait(int fmt, int nt, bool deep, int c, int ahead) {
+  const int hu0 = fmt == 0 ? 3 * nt : 8 * nt, u1 = fmt == 0 ? 2 * nt : 6 * nt;
+  int n = 0;
+  for (int k = 0; k < ahead; ++k) {  // stage s - k; the DMA of stage s + 1 went out at k = ahead - 1
+    const int st = (c - k + 8) & 3;
+    if (k + 1 < ahead) n += 4;
+    n += deep ? (st == 0 ? hu0 + u1 : 0) : st == 0 ? u1 : st == 2 ? hu0 : 0;
+  }
+  return n > 63 ? 63 : n;
 }
-template <int FMT, int WPE, int NTW>
+template <int FMT, int WPE, int NTW, bool DEEP>
 __global__ __launch_bounds__(64 * kGemmWaves) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void quant_gemm32s_kernel(
     const uint8_t *__restrict__ W, const uint4 *__restrict__ xa,
     const float *__restrict__ tscale, float *__restrict__ Y, int N,
     int M, int nblk, int ntiles, int MTG, int F, int S, int R, float *__restrict__ part) {
   constexpr int NW = kGemmWaves;
   constexpr int kUnits = kQ4kRecord / 16;                       // 144 units per Q4_K record
-  constexpr int kSU = 4 * 2 * 64;                               // 512 units (8 KB) per stage
+  constexpr int kSU = 4 * 4 * 64;                               // 1024 units (16 KB) per stage
+  constexpr int NB = DEEP || NTW == 2 ? 4 : 2, AH = NB - 1;
   constexpr int NT = NTW;                                       // 32-row MFMA tiles per wave
   constexpr int kBTn = 2 * NT * NW;                             // 16-row tiles per workgroup
   constexpr int kRT = 16 * kBTn;                                // rows per workgroup tile
@@ -539,8 +548,8 @@ __global__ __launch_bounds__(64 * kGemmWaves) __attribute__((amdgpu_waves_per_eu
   // of one stage does not wait for the DMA into another.
   __shared__ u32x4 As0[kSU];
   __shared__ u32x4 As1[kSU];
-  __shared__ u32x4 As2[kSU];
-  __shared__ u32x4 As3[kSU];
+  __shared__ u32x4 As2[NB > 2 ? kSU : 1];
+  __shared__ u32x4 As3[NB > 3 ? kSU : 1];
   __shared__ __align__(16) float ts_lds[kBM];  // the token scales of this token tile
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -560,15 +569,12 @@ __global__ __launch_bounds__(64 * kGemmWaves) __attribute__((amdgpu_waves_per_eu
   const int tile0 = kBTn * ng;
   // Stage s = 8 b + 2 c + h: slices 16 (4 b + c) + h + 2 hi of token tile i at [(2 i + hi) * 64],
   // one 1 KB wave load each; wave w loads units kDMA w .. kDMA w + kDMA - 1 (unit 2 i + hi).
-  auto load_stage = [&](int s, u32x4 *dst) {
-    const int ch = 4 * kb0 + (s >> 1), h = s & 1;  // s counts from the range start
+  const void *abase = xg;
+  const int off16 = 16 * lane;
+  auto load_stage = [&](int s, u32x4 *dst) {  // chunk s of the range: wave w loads token tile w's 4 K16 slices
+    const int so = (4 * kb0 + s) * 4096 + wave * nq * 1024;
 #pragma unroll
-    for (int j = 0; j < kDMA; ++j) {
-      const int p = kDMA * wave + j, i = p >> 1, hi = p & 1;
-      __builtin_amdgcn_global_load_lds(
-          (const void *)(xg + ((size_t)i * nq + 4 * ch + h + 2 * hi) * 64 + lane),
-          (__attribute__((address_space(3))) void *)(dst + (2 * i + hi) * 64), 16, 0, 0);
-    }
+    for (int j = 0; j < 4; ++j) lds_load16(abase, dst + (4 * wave + j) * 64, off16, so + j * 1024);
   };
   auto buf = [&](int k) -> u32x4 * { return k == 0 ? As0 : k == 1 ? As1 : k == 2 ? As2 : As3; };
 
@@ -588,47 +594,50 @@ __global__ __launch_bounds__(64 * kGemmWaves) __attribute__((amdgpu_waves_per_eu
     return W + ((size_t)min(tile0 + tl(t), ntiles - 1) * nblk + b) * kQ6kRecord;
   };
   auto nib = [&](int c2, int h) { return kQ4kHdr / 16 + 64 * c2 + 16 * (2 * h + kap) + r16; };
-  u32x4 hdr[NT], u0[NT][2], u1[NT][2];    // Q4_K
-  uint2 ql6[NT][2][4], qh6[NT][2][2];     // Q6_K: [half][group], [half][K16 half]
-  uint32_t dw6[NT];                       // Q6_K: the row's d (f16 bits)
-  auto load_hu0 = [&](int b) {
+  // DEEP: two slots, a whole super-block loaded one ahead; else slot 0, each part reloaded once its
+  // last use has been read out.
+  constexpr int NS = DEEP ? 2 : 1;
+  u32x4 hdr[NS][NT], u0[NS][NT][2], u1[NS][NT][2];  // Q4_K
+  uint2 ql6[NS][NT][2][4], qh6[NS][NT][2][2];       // Q6_K: [half][group], [half][K16 half]
+  uint32_t dw6[NS][NT];                             // Q6_K: the row's d (f16 bits)
+  auto load_hu0 = [&](int b, int sl) {
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       if (FMT == 0) {
         const u32x4 *r = rec(t, b);
-        hdr[t] = r[r16];
-        u0[t][0] = r[nib(0, 0)];
-        u0[t][1] = r[nib(0, 1)];
+        hdr[sl][t] = r[r16];
+        u0[sl][t][0] = r[nib(0, 0)];
+        u0[sl][t][1] = r[nib(0, 1)];
       } else {
         const uint8_t *r = rec6(t, b);
-        hdr[t] = *reinterpret_cast<const u32x4 *>(r + 16 * r16);
-        dw6[t] = *reinterpret_cast<const uint16_t *>(r + kQ6kD + 2 * r16);
+        hdr[sl][t] = *reinterpret_cast<const u32x4 *>(r + 16 * r16);
+        dw6[sl][t] = *reinterpret_cast<const uint16_t *>(r + kQ6kD + 2 * r16);
 #pragma unroll
         for (int g = 0; g < 4; ++g)
-          ql6[t][0][g] = *reinterpret_cast<const uint2 *>(r + kQ6kQl + 16 * (16 * g + r16) + 8 * kap);
+          ql6[sl][t][0][g] = *reinterpret_cast<const uint2 *>(r + kQ6kQl + 16 * (16 * g + r16) + 8 * kap);
 #pragma unroll
         for (int h = 0; h < 2; ++h)
-          qh6[t][0][h] = *reinterpret_cast<const uint2 *>(r + kQ6kQh + 256 * h + 16 * r16 + 8 * kap);
+          qh6[sl][t][0][h] = *reinterpret_cast<const uint2 *>(r + kQ6kQh + 256 * h + 16 * r16 + 8 * kap);
       }
     }
   };
-  auto load_u1 = [&](int b) {
+  auto load_u1 = [&](int b, int sl) {
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       if (FMT == 0) {
         const u32x4 *r = rec(t, b);
-        u1[t][0] = r[nib(1, 0)];
-        u1[t][1] = r[nib(1, 1)];
+        u1[sl][t][0] = r[nib(1, 0)];
+        u1[sl][t][1] = r[nib(1, 1)];
       } else {
         const uint8_t *r = rec6(t, b);
 #pragma unroll
         for (int g = 0; g < 4; ++g)
-          ql6[t][1][g] = *reinterpret_cast<const uint2 *>(r + kQ6kQl + 1024 + 16 * (16 * g + r16) +
-                                                          8 * kap);
+          ql6[sl][t][1][g] = *reinterpret_cast<const uint2 *>(r + kQ6kQl + 1024 + 16 * (16 * g + r16) +
+                                                              8 * kap);
 #pragma unroll
         for (int h = 0; h < 2; ++h)
-          qh6[t][1][h] = *reinterpret_cast<const uint2 *>(r + kQ6kQh + 512 + 256 * h + 16 * r16 +
-                                                          8 * kap);
+          qh6[sl][t][1][h] = *reinterpret_cast<const uint2 *>(r + kQ6kQh + 512 + 256 * h + 16 * r16 +
+                                                              8 * kap);
       }
     }
   };
@@ -641,35 +650,38 @@ __global__ __launch_bounds__(64 * kGemmWaves) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
-  const int nstage = (kb1 - kb0) * 8;
-  // Issue order as in the loop below at the start of a super-block: header and chunk 0-1
-  // units, then stages 0-2.
-  load_hu0(kb0);
-  load_stage(0, As0);
-  load_stage(1, As1);
-  load_stage(2, As2);
+  const int nstage = (kb1 - kb0) * 4;
+  load_hu0(kb0, 0);
+  if (DEEP) load_u1(kb0, 0);
+#pragma unroll
+  for (int k = 0; k < AH; ++k) load_stage(k, buf(k));
   for (int k = tid; k < kBM; k += 64 * NW) ts_lds[k] = tscale[kBM * mg + k];  // MTG * kBM entries
-  FHIP_LDS_BARRIER(wait_vm(2 * kDMA));
+  FHIP_LDS_BARRIER(wait_vm(0));
+  const uint32_t al = in_reg(lane);
 
   // A record register enters the arithmetic through an empty asm at the stage that first uses
   // it: the compiler would otherwise hoist the dequantization next to the load and wait for it
   // there (vmcnt(0)), with the registers of both held at once.
   auto pin = [](u32x4 &v) { asm volatile("" : "+v"(v)); };
   auto pin2 = [](uint2 &v) { asm volatile("" : "+v"(v.x), "+v"(v.y)); };
-  for (int b = kb0; b < kb1; ++b) {
+  // LAST (DEEP only): the range's last super-block, with no record to load ahead (the compiler would
+  // drop such loads, and the waits count them).
+  auto super_block = [&](int b, auto slot, auto last) {
+    constexpr int sl = decltype(slot)::value;
+    constexpr bool LAST = decltype(last)::value;
     RowScales rs[NT];
     uint32_t sc6[NT][4];  // Q6_K: the row's 16 int8 scales, one word per chunk
     float d6[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      pin(hdr[t]);
+      pin(hdr[sl][t]);
       if (FMT == 0) {
-        rs[t] = row_scales(__builtin_bit_cast(uint4, hdr[t]), K);
+        rs[t] = row_scales(__builtin_bit_cast(uint4, hdr[sl][t]), K);
       } else {
-        asm volatile("" : "+v"(dw6[t]));
+        asm volatile("" : "+v"(dw6[sl][t]));
 #pragma unroll
-        for (int j = 0; j < 4; ++j) sc6[t][j] = hdr[t][j];
-        d6[t] = (float)__builtin_bit_cast(_Float16, (uint16_t)dw6[t]);
+        for (int j = 0; j < 4; ++j) sc6[t][j] = hdr[sl][t][j];
+        d6[t] = (float)__builtin_bit_cast(_Float16, (uint16_t)dw6[sl][t]);
       }
     }
 #pragma unroll
@@ -679,12 +691,12 @@ __global__ __launch_bounds__(64 * kGemmWaves) __attribute__((amdgpu_waves_per_eu
         for (int t = 0; t < NT; ++t) {
           if (FMT == 0) {
 #pragma unroll
-            for (int h = 0; h < 2; ++h) pin(c == 0 ? u0[t][h] : u1[t][h]);
+            for (int h = 0; h < 2; ++h) pin(c == 0 ? u0[sl][t][h] : u1[sl][t][h]);
           } else {
 #pragma unroll
-            for (int g = 0; g < 4; ++g) pin2(ql6[t][c >> 1][g]);
+            for (int g = 0; g < 4; ++g) pin2(ql6[sl][t][c >> 1][g]);
 #pragma unroll
-            for (int h = 0; h < 2; ++h) pin2(qh6[t][c >> 1][h]);
+            for (int h = 0; h < 2; ++h) pin2(qh6[sl][t][c >> 1][h]);
           }
         }
       uint2 xb[NT][2];  // Q4_K: nibble bytes of lane group g = 2 h + kap of chunk c
@@ -693,21 +705,26 @@ __global__ __launch_bounds__(64 * kGemmWaves) __attribute__((amdgpu_waves_per_eu
         for (int t = 0; t < NT; ++t)
 #pragma unroll
           for (int h = 0; h < 2; ++h) {
-            const u32x4 v = c < 2 ? u0[t][h] : u1[t][h];
+            const u32x4 v = c < 2 ? u0[sl][t][h] : u1[sl][t][h];
             xb[t][h] = (c & 1) ? make_uint2(v[2], v[3]) : make_uint2(v[0], v[1]);
           }
       }
+      load_stage(min(4 * (b - kb0) + c + AH, nstage - 1), buf((c + AH) % NB));
+      // The waits count on the records behind the stage's DMA: no load is scheduled across.
+      __builtin_amdgcn_sched_barrier(kNoLoadAcross);
+      if (DEEP) {
+        if (c == 0 && !LAST) {
+          load_hu0(min(b + 1, kb1 - 1), sl ^ 1);
+          load_u1(min(b + 1, kb1 - 1), sl ^ 1);
+        }
+      } else {
+        if (c == 0) load_u1(b, 0);
+        if (c == 2) load_hu0(min(b + 1, kb1 - 1), 0);
+      }
+      __builtin_amdgcn_sched_barrier(kNoLoadAcross);
+      const u32x4 *Acur = buf(c % NB);
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const int ls = 2 * c + h;  // stage within the super-block (its buffer is ls & 3)
-        const int s = 8 * (b - kb0) + ls;
-        load_stage(min(s + 3, nstage - 1), buf((ls + 3) & 3));
-        // Each record register is reloaded once its last use has been read out: chunk 2-3
-        // units of this super-block at stage 0 (used from stage 4), header and chunk 0-1 units
-        // of the next one at stage 4 (used from its stage 0).
-        if (ls == 0) load_u1(b);
-        if (ls == 4) load_hu0(min(b + 1, kb1 - 1));
-        const u32x4 *Acur = buf(ls & 3);
         f16x8 bl[NT], bh[NT];
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
@@ -718,7 +735,7 @@ __global__ __launch_bounds__(64 * kGemmWaves) __attribute__((amdgpu_waves_per_eu
             // half's ql bytes, 2-bit fields of its qh bytes; scales of sub-blocks 4c + h, 4c + 2 + h
             uint32_t scw = sc6[t][c];
             float dd6 = d6[t];
-            uint2 qa = ql6[t][c >> 1][h], qb = ql6[t][c >> 1][2 + h], qhh = qh6[t][c >> 1][h];
+            uint2 qa = ql6[sl][t][c >> 1][h], qb = ql6[sl][t][c >> 1][2 + h], qhh = qh6[sl][t][c >> 1][h];
             pin2(qa); pin2(qb); pin2(qhh);
             asm volatile("" : "+v"(scw), "+v"(dd6));
             const _Float16 Sa = (_Float16)(dd6 * (float)(int8_t)(scw >> (8 * h)));
@@ -731,7 +748,7 @@ __global__ __launch_bounds__(64 * kGemmWaves) __attribute__((amdgpu_waves_per_eu
         for (int hi = 0; hi < 2; ++hi) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const f16x8 a = __builtin_bit_cast(f16x8, Acur[(2 * i + hi) * 64 + lane]);
+            const f16x8 a = __builtin_bit_cast(f16x8, Acur[(4 * i + 2 * hi + h) * 64 + al]);
 #pragma unroll
             for (int t = 0; t < NT; ++t)
               acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, hi ? bh[t] : bl[t], acc[i][t], 0, 0, 0);
@@ -742,21 +759,26 @@ __global__ __launch_bounds__(64 * kGemmWaves) __attribute__((amdgpu_waves_per_eu
           // before), and 64 rows per wave fit 256 VGPRs without a spill.
           if ((FMT == 1 || NT == 2) && hi == 0) __builtin_amdgcn_sched_barrier(0);
         }
-        // Stage s + 1 has landed (for every wave, after the barrier) once at most stages s + 2
-        // and s + 3 (kDMA loads each) and the record loads that gemm32s_wait allows are
-        // pending.
-        switch (ls) {
-          case 0: FHIP_LDS_BARRIER(wait_vm(gemm32s_wait(FMT, NT, 0, kDMA))); break;
-          case 1: FHIP_LDS_BARRIER(wait_vm(gemm32s_wait(FMT, NT, 1, kDMA))); break;
-          case 2: FHIP_LDS_BARRIER(wait_vm(gemm32s_wait(FMT, NT, 2, kDMA))); break;
-          case 3: FHIP_LDS_BARRIER(wait_vm(gemm32s_wait(FMT, NT, 3, kDMA))); break;
-          case 4: FHIP_LDS_BARRIER(wait_vm(gemm32s_wait(FMT, NT, 4, kDMA))); break;
-          case 5: FHIP_LDS_BARRIER(wait_vm(gemm32s_wait(FMT, NT, 5, kDMA))); break;
-          case 6: FHIP_LDS_BARRIER(wait_vm(gemm32s_wait(FMT, NT, 6, kDMA))); break;
-          default: FHIP_LDS_BARRIER(wait_vm(gemm32s_wait(FMT, NT, 7, kDMA))); break;
-        }
+      }
+      switch (c) {
+        case 0: FHIP_LDS_BARRIER(wait_vm(LAST ? 4 * (AH - 1) : gemm32s_wait(FMT, NT, DEEP, 0, AH))); break;
+        case 1: FHIP_LDS_BARRIER(wait_vm(LAST ? 4 * (AH - 1) : gemm32s_wait(FMT, NT, DEEP, 1, AH))); break;
+        case 2: FHIP_LDS_BARRIER(wait_vm(LAST ? 4 * (AH - 1) : gemm32s_wait(FMT, NT, DEEP, 2, AH))); break;
+        default: FHIP_LDS_BARRIER(wait_vm(LAST ? 4 * (AH - 1) : gemm32s_wait(FMT, NT, DEEP, 3, AH))); break;
       }
     }
+  };
+  // Pairs without a branch between them: a load in flight for the second super-block would be moved
+  // down to it.
+  int b = kb0;
+  if constexpr (DEEP) {
+    for (; b + 2 <= kb1; b += 2) {
+      super_block(b, std::integral_constant<int, 0>{}, std::false_type{});
+      super_block(b + 1, std::integral_constant<int, 1>{}, std::false_type{});
+    }
+    if (b < kb1) super_block(b, std::integral_constant<int, 0>{}, std::true_type{});
+  } else {
+    for (; b < kb1; ++b) super_block(b, std::integral_constant<int, 0>{}, std::false_type{});
   }
   __builtin_amdgcn_s_waitcnt(wait_vm(0));  // no LDS DMA may be pending when the workgroup ends
 
@@ -839,6 +861,7 @@ namespace {
 // token scales, then the K-range partial results).
 struct GemmPlan {
   int MTG, tasks, form, F, S, R;  // tile tasks; F whole, then R split into S K ranges each
+  bool deep;                      // a super-block of records loaded one ahead
   int nt;                         // 32-row MFMA tiles per wave: 1 (128-row tiles) or 2 (256)
   size_t xab, tsb, pb;
 };
@@ -902,6 +925,12 @@ GemmPlan plan_gemm32(int fmt, int N, int K, int M) {
       p.F = p.tasks - R;
     }
   }
+  // Q4_K loads whole super-blocks of records one ahead (two workgroups per CU) while the grid gives a
+  // CU about that many: us, three workgroups per CU / this, 256 tokens of 18944 x 3584 54.6 / 50.3, of
+  // 25600 x 5120 86.6 / 81.9, 896 of 3584 x 18944 179 / 171; 512 of 18944 x 3584 (592 tiles) 82.6 /
+  // 84.5, of 25600 x 5120 (800) 145.8 / 147.9. Q6_K, whose records take 14 loads, is no faster so
+  // (512 tokens of 18944 x 3584 94.0 / 99.3).
+  p.deep = fmt == 0 && p.tasks < 2 * cus;
   p.xab = ((size_t)p.MTG * kBM * K * 2 + 255) & ~(size_t)255;
   p.tsb = ((size_t)p.MTG * kBM * 4 + 255) & ~(size_t)255;
   p.pb = p.R ? (size_t)(p.S - 1) * p.R * kTileElems * p.nt * 4 : 0;
@@ -938,10 +967,10 @@ int launch_gemm32(int fmt, const void *Wv, const float *X, float *Y, int N, int 
   const int grid2 = p.F + p.R * p.S;
   if (fmt == 1 && p.form != 1) {
     if (p.nt == 2)
-      quant_gemm32s_kernel<1, 2, 2><<<grid2, 64 * kGemmWaves, 0, stream()>>>(
+      quant_gemm32s_kernel<1, 2, 2, false><<<grid2, 64 * kGemmWaves, 0, stream()>>>(
           W, xa, ts, Y, N, M, nblk, ntiles, MTG, p.F, p.S, p.R, part);
     else
-      quant_gemm32s_kernel<1, 3, 1><<<grid2, 64 * kGemmWaves, 0, stream()>>>(
+      quant_gemm32s_kernel<1, 3, 1, false><<<grid2, 64 * kGemmWaves, 0, stream()>>>(
           W, xa, ts, Y, N, M, nblk, ntiles, MTG, p.F, p.S, p.R, part);
     FHIP_CHECK_LAUNCH("quant_gemm32s_kernel<1>");
     return reduce();
@@ -954,10 +983,13 @@ int launch_gemm32(int fmt, const void *Wv, const float *X, float *Y, int N, int 
   }
   if (p.form != 1) {
     if (p.nt == 2)
-      quant_gemm32s_kernel<0, 2, 2><<<grid2, 64 * kGemmWaves, 0, stream()>>>(
+      quant_gemm32s_kernel<0, 2, 2, false><<<grid2, 64 * kGemmWaves, 0, stream()>>>(
+          W, xa, ts, Y, N, M, nblk, ntiles, MTG, p.F, p.S, p.R, part);
+    else if (p.deep)
+      quant_gemm32s_kernel<0, 2, 1, true><<<grid2, 64 * kGemmWaves, 0, stream()>>>(
           W, xa, ts, Y, N, M, nblk, ntiles, MTG, p.F, p.S, p.R, part);
     else
-      quant_gemm32s_kernel<0, 3, 1><<<grid2, 64 * kGemmWaves, 0, stream()>>>(
+      quant_gemm32s_kernel<0, 3, 1, false><<<grid2, 64 * kGemmWaves, 0, stream()>>>(
           W, xa, ts, Y, N, M, nblk, ntiles, MTG, p.F, p.S, p.R, part);
     FHIP_CHECK_LAUNCH("quant_gemm32s_kernel<0>");
     return reduce();
