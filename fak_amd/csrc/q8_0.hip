@@ -442,6 +442,11 @@ int fhip_q8_0_matmul_f32(const void *dPacked, const float *dX, float *dY, int ou
     return fail(FHIP_EINVAL, "fhip_q8_0_matmul_f32: dX and dPacked must be 16-byte aligned");
   if (int rc = check_weight("fhip_q8_0_matmul_f32", dPacked, kWeightQ8_0, out, in)) return rc;
   untag_range(dY, (size_t)P * out * 4);
+  if (in > 1 << 21) {  // the GEMM's operand offsets are 32-bit: such rows go token by token
+    for (int t = 0; t < P; ++t)
+      if (int rc = q8_0_gemv(dPacked, dX + (size_t)t * in, dY + (size_t)t * out, out, in, 1)) return rc;
+    return FHIP_OK;
+  }
   if (q8_takes_gemv(out, in, P)) return q8_0_gemv(dPacked, dX, dY, out, in, P);
   for (int t0 = 0; t0 < P; t0 += kQ8GemmTokens) {
     const int m = P - t0 < kQ8GemmTokens ? P - t0 : kQ8GemmTokens;
