@@ -28,7 +28,7 @@
 //     adds them after a barrier, in record order. A window's terms must fit in LDS; long rows or
 //     many tokens take several windows, the sums carrying across.
 // Weight records stream through a ring of PF in-flight loads per wave (three 16-byte loads per
-// lane per record), as in the Q4_K GEMV.
+// lane per record), as in the Q4_K GEMV. One token has a kernel of its own (q4k_i8route1_kernel).
 #include "kernels.hpp"
 #include "q8round.hpp"
 
@@ -310,6 +310,151 @@ __global__ __launch_bounds__(512) void q4k_i8route_kernel(
   }
 }
 
+// One token. The general kernel below spends a 16-token matrix instruction and every lane's term
+// arithmetic on a token that a quarter of the lanes hold; here
+//   * one chained v_mfma_i32_16x16x64_i8 result per record holds the eight sub-block sums: sub-block s
+//     owns operand row 4 (s / 2) + s % 2 (the other rows are zero), so result lane (g, r) holds I of
+//     sub-blocks 2g and 2g + 1 of row r and forms their four terms only;
+//   * the terms of the whole K go to LDS, by KW waves per tile in parallel, and after one barrier a
+//     lane per row adds them in order: the reference's chain at the latency of its additions;
+//   * each workgroup quantizes the activation itself, eight lanes per block, under its first records.
+// VALU per record ~110 against ~300. us: 18944 x 3584 17.4 -> 11.9-12.6 (38.3 MB: 7.6 us at a
+// large copy's rate), 3584 x 3584 9.9 -> 7.1, 3584 x 18944 23.0 -> 17.9, 152064 x 3584 87.4 -> 63.7.
+constexpr int kOnePF = 4;  // records in flight per wave
+__host__ __device__ inline size_t i8r1_lds(int nblk, int TW) {
+  return (size_t)nblk * (256 + 64) + (size_t)TW * nblk * 1024;  // codes, {S, dx}, terms
+}
+
+__global__ __launch_bounds__(1024) void q4k_i8route1_kernel(const uint8_t *__restrict__ W,
+                                                            const float *__restrict__ X,
+                                                            float *__restrict__ Y, int N, int nblk,
+                                                            int ntiles, int KW, int TW) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  uint8_t *codes = smem;
+  float2 *sd = reinterpret_cast<float2 *>(smem + 256 * nblk);
+  float4 *terms = reinterpret_cast<float4 *>(smem + 320 * nblk);
+  const int tid = threadIdx.x, lane = tid & 63, nthr = blockDim.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tile = wave / KW, part = wave - tile * KW;
+  const int T = blockIdx.x * TW + tile;
+  const int g = lane >> 4, r = lane & 15;
+  const int p0 = part * nblk / KW, p1 = (part + 1) * nblk / KW;  // this wave's records (may be none)
+  const uint8_t *base = W + (size_t)min(T, ntiles - 1) * nblk * kQ4kRecord;
+
+  // Activation loads first (vector loads complete in issue order), then the first records.
+  constexpr int XI = 4;
+  const int nx = 64 * nblk;  // float4 units
+  const float4 *X4 = reinterpret_cast<const float4 *>(X);
+  float4 xv[XI];
+#pragma unroll
+  for (int i = 0; i < XI; ++i) xv[i] = X4[min(tid + nthr * i, nx - 1)];
+  uint4 rh[kOnePF], ra[kOnePF], rb[kOnePF];
+  auto load = [&](int b, int u) {
+    const uint8_t *rec = base + (size_t)min(b, nblk - 1) * kQ4kRecord;
+    rh[u] = ld_stream(rec + 16 * r);
+    ra[u] = ld_stream(rec + kQ4kHdr + 16 * lane);
+    rb[u] = ld_stream(rec + kQ4kHdr + 1024 + 16 * lane);
+  };
+#pragma unroll
+  for (int u = 0; u < kOnePF; ++u) load(min(p0 + u, max(p1, 1) - 1), u);
+  // quantizeRowQ8scalar of four values: lanes 8k .. 8k + 7 hold a block, valid together.
+  auto quantize = [&](int v, const float4 x) {
+    float amax = fmaxf(fmaxf(fmaxf(fmaxf(0.f, fabsf(x.x)), fabsf(x.y)), fabsf(x.z)), fabsf(x.w));
+    amax = fmaxf(amax, __shfl_xor(amax, 1));
+    amax = fmaxf(amax, __shfl_xor(amax, 2));
+    amax = fmaxf(amax, __shfl_xor(amax, 4));
+    const float d = __fdiv_rn(amax, 127.f);
+    int c0 = 0, c1 = 0, c2 = 0, c3 = 0;
+    if (d != 0.f) {
+      const float inv = __fdiv_rn(1.f, d);
+      c0 = q8round(__fmul_rn(x.x, inv));
+      c1 = q8round(__fmul_rn(x.y, inv));
+      c2 = q8round(__fmul_rn(x.z, inv));
+      c3 = q8round(__fmul_rn(x.w, inv));
+    }
+    int sum = c0 + c1 + c2 + c3;
+    sum += __shfl_xor(sum, 1);
+    sum += __shfl_xor(sum, 2);
+    sum += __shfl_xor(sum, 4);
+    if (v < nx) {
+      *reinterpret_cast<uint32_t *>(codes + 4 * v) =
+          (uint32_t)(c0 & 255) | (uint32_t)(c1 & 255) << 8 | (uint32_t)(c2 & 255) << 16 | (uint32_t)c3 << 24;
+      if ((v & 7) == 0) sd[v >> 3] = make_float2((float)sum, d);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < XI; ++i) quantize(tid + nthr * i, xv[i]);
+  for (int v = tid + nthr * XI; v - tid < nx; v += nthr) quantize(v, X4[min(v, nx - 1)]);
+  __syncthreads();
+
+  // Operand rows: lane row r owns sub-block 2 (r / 4) + r % 2 when r % 4 < 2, in the chunk r / 4; its
+  // eight codes sit in the half of the operand that its sub-block's nibbles take.
+  const bool own = (r & 3) < 2;
+  const uint8_t *cp = codes + 32 * (2 * (r >> 2) + (r & 1)) + 8 * g;
+  const uint32_t mlo = own && !(r & 1) ? ~0u : 0u, mhi = own && (r & 1) ? ~0u : 0u;
+  uint32_t mc[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) mc[c] = (r >> 2) == c ? ~0u : 0u;
+  const uint32_t k0F = 0x0F0F0F0Fu;
+  float4 *tw = terms + (size_t)tile * nblk * 64 + 4 * r + (g ^ (r >> 2));
+  for (int bb = p0; bb < p1; bb += kOnePF) {
+#pragma unroll
+    for (int u = 0; u < kOnePF; ++u) {
+      const int b = bb + u;
+      if (b >= p1) break;
+      const uint2 cv = *reinterpret_cast<const uint2 *>(cp + 256 * b);
+      const uint32_t a0 = cv.x & mlo, a1 = cv.y & mlo, a2 = cv.x & mhi, a3 = cv.y & mhi;
+      const uint32_t q[8] = {ra[u].x, ra[u].y, ra[u].z, ra[u].w, rb[u].x, rb[u].y, rb[u].z, rb[u].w};
+      i32x4 D = {0, 0, 0, 0};
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const uint32_t w0 = q[2 * c], w1 = q[2 * c + 1];
+        const i32x4 A = {(int)(a0 & mc[c]), (int)(a1 & mc[c]), (int)(a2 & mc[c]), (int)(a3 & mc[c])};
+        const i32x4 B = {(int)(w0 & k0F), (int)(w1 & k0F), (int)((w0 >> 4) & k0F), (int)((w1 >> 4) & k0F)};
+        D = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, B, D, 0, 0, 0);
+      }
+      const uint4 h = rh[u];
+      const float d = (float)__builtin_bit_cast(_Float16, (uint16_t)(h.x & 0xffffu));
+      const float dmin = (float)__builtin_bit_cast(_Float16, (uint16_t)(h.x >> 16));
+      // GetScaleMinK4 of sub-blocks 2g and 2g + 1: bytes 2 (g % 2) and the next of the low or high four.
+      uint32_t sc = g < 2 ? h.y & 0x3F3F3F3Fu : (h.w & k0F) | ((h.y >> 2) & 0x30303030u);
+      uint32_t mn = g < 2 ? h.z & 0x3F3F3F3Fu : ((h.w >> 4) & k0F) | ((h.z >> 2) & 0x30303030u);
+      sc >>= 16 * (g & 1);
+      mn >>= 16 * (g & 1);
+      const float4 e = *reinterpret_cast<const float4 *>(sd + 8 * b + 2 * g);  // {S, dx} of both
+      float4 t;
+      t.x = __fmul_rn(__fmul_rn((float)D[0], __fmul_rn(d, (float)(sc & 255))), e.y);
+      t.y = __fmul_rn(__fmul_rn(e.x, __fmul_rn(dmin, (float)(mn & 255))), e.y);
+      t.z = __fmul_rn(__fmul_rn((float)D[1], __fmul_rn(d, (float)((sc >> 8) & 255))), e.w);
+      t.w = __fmul_rn(__fmul_rn(e.z, __fmul_rn(dmin, (float)((mn >> 8) & 255))), e.w);
+      tw[64 * b] = t;
+      load(min(b + kOnePF, p1 - 1), u);
+    }
+  }
+  __syncthreads();
+  if (part != 0 || lane >= 16) return;
+  const float4 *tr = terms + (size_t)tile * nblk * 64 + 4 * r;
+  const int f = r >> 2;
+  float acc = 0.f;
+  auto add = [&](const float4 t) {
+    acc = __fsub_rn(__fadd_rn(acc, t.x), t.y);
+    acc = __fsub_rn(__fadd_rn(acc, t.z), t.w);
+  };
+  int b = 0;
+  for (; b + 2 <= nblk; b += 2) {  // eight reads in flight per pair of records
+    float4 t[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) t[k] = tr[64 * (b + (k >> 2)) + ((k & 3) ^ f)];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) add(t[k]);
+  }
+  for (; b < nblk; ++b)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) add(tr[64 * b + (k ^ f)]);
+  const int row = 16 * T + r;
+  if (T < ntiles && row < N) Y[row] = acc;
+}
+
 }  // namespace
 }  // namespace fhip
 
@@ -330,6 +475,28 @@ extern "C" int fhip_q4k_matmul_int8_f32(const void *dPacked, const float *dX, fl
   if (int rc = check_weight("fhip_q4k_matmul_int8_f32", dPacked, kWeightQ4K, out, in)) return rc;
   untag_range(dY, (size_t)P * out * 4);
   const int nblk = in / 256;
+  const int ntiles = q4k_tiles(out);
+  // One token, except on the widest matrices' long rows, whose parked terms leave a CU too few waves
+  // where the general kernel's eight-tile workgroups park none (us, one-token / general: 25600 x 4096
+  // 17.8 / 18.4, 25600 x 5120 23.0 / 20.9, 152064 x 3584 63.9 / 87.4, 152064 x 5120 127 / 101, 16384 x
+  // 11008 57 / 40).
+  if (P == 1 && tuning().i8r_kw <= 0 && tuning().i8r_tw <= 0 && (ntiles < 4 * cu_count() || nblk <= 16) &&
+      i8r1_lds(nblk, 1) <= (size_t)lds_limit()) {
+    // Waves per tile until the grid has eight per CU (each at least a record) and the workgroups that fit
+    // a CU's LDS have twelve, then tiles per workgroup,
+    // which share its quantized activation, up to four waves while the grid covers the CUs twice and
+    // two workgroups' terms fit in LDS. us at waves x tiles: 18944 x 3584 2 x 2 12.8, 4 x 1 14.1, 4 x 2
+    // 16.4, 1 x 4 13.8; 152064 x 3584 1 x 4 64, 2 x 2 65, 4 x 1 83; 3584 x 18944 16 x 1 18.2, 8 x 1 20.0.
+    const int cus = cu_count() > 0 ? cu_count() : 256;
+    int KW = 1, TW = 1;
+    const int fit = (int)((size_t)lds_limit() / i8r1_lds(nblk, 1));
+    while (KW < 16 && ((long long)ntiles * KW < 8LL * cus || KW * fit < 12) && 2 * KW <= nblk) KW *= 2;
+    while (2 * TW * KW <= 4 && i8r1_lds(nblk, 2 * TW) <= (size_t)lds_limit() / 2 && ntiles >= 4 * TW * cus) TW *= 2;
+    q4k_i8route1_kernel<<<ceil_div(ntiles, TW), 64 * KW * TW, i8r1_lds(nblk, TW), stream()>>>(
+        reinterpret_cast<const uint8_t *>(dPacked), dX, dY, out, nblk, ntiles, KW, TW);
+    FHIP_CHECK_LAUNCH("q4k_i8route1_kernel");
+    return FHIP_OK;
+  }
   const bool fused = P <= kFusedTokens;
   int8_t *qx = nullptr;
   float2 *sdg = nullptr;
@@ -351,7 +518,6 @@ extern "C" int fhip_q4k_matmul_int8_f32(const void *dPacked, const float *dX, fl
   // whose LDS fits the device. (One token with ~16 waves per CU put 4 waves on each 18944 x 3584
   // tile: 26.2 us against 21.4 with 2; the 3584 x 18944 down projection keeps 8 either way.
   // Eight tokens on 18944 x 3584 want 4: 91 us, 130 with 2.)
-  const int ntiles = q4k_tiles(out);
   const int groups = ceil_div(P, kTokGroup);
   const int pg = P < kTokGroup ? P : kTokGroup;
   int KW = tuning().i8r_kw, TW = 1;
