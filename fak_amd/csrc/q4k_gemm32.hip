@@ -723,6 +723,18 @@ __global__ __launch_bounds__(64 * kGemmWaves) __attribute__((amdgpu_waves_per_eu
       }
       __builtin_amdgcn_sched_barrier(kNoLoadAcross);
       const u32x4 *Acur = buf(c % NB);
+      // 64 rows per wave of Q4_K: the operand reads run AR ahead of their MFMAs, which nothing but ALU
+      // instructions may pass (the compiler read two and waited for them: 2048 tokens of 18944 x 3584
+      // 267 -> 261 us; no gain at 32 rows per wave or Q6_K).
+      constexpr int AR = FMT == 0 && NT == 2 ? 3 : 0;
+      f16x8 fr[AR + 1];
+      auto rd = [&](int f) {  // fragment f: h = f / 8, K16 half f / 4 % 2, token tile f % 4
+        return __builtin_bit_cast(f16x8, Acur[(4 * (f & 3) + 2 * ((f >> 2) & 1) + (f >> 3)) * 64 + al]);
+      };
+      if (AR > 0) {
+#pragma unroll
+        for (int f = 0; f < AR; ++f) fr[f] = rd(f);
+      }
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         f16x8 bl[NT], bh[NT];
@@ -748,16 +760,19 @@ __global__ __launch_bounds__(64 * kGemmWaves) __attribute__((amdgpu_waves_per_eu
         for (int hi = 0; hi < 2; ++hi) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const f16x8 a = __builtin_bit_cast(f16x8, Acur[(4 * i + 2 * hi + h) * 64 + al]);
+            const int f = 8 * h + 4 * hi + i;
+            if (f + AR < 16) fr[(f + AR) % (AR + 1)] = rd(f + AR);
+            const f16x8 a = fr[f % (AR + 1)];
 #pragma unroll
             for (int t = 0; t < NT; ++t)
               acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, hi ? bh[t] : bl[t], acc[i][t], 0, 0, 0);
+            if (AR > 0) __builtin_amdgcn_sched_barrier(0x6);
           }
-          // Q6_K, and 64 rows per wave: the second K16 half's operand reads wait for the first
-          // half's MFMAs (and Q6_K's code words enter each stage through fresh pinned copies):
-          // so scheduled Q6_K needs 145 VGPRs and runs three workgroups per CU (219, and two,
-          // before), and 64 rows per wave fit 256 VGPRs without a spill.
-          if ((FMT == 1 || NT == 2) && hi == 0) __builtin_amdgcn_sched_barrier(0);
+          // Q6_K: the second K16 half's operand reads wait for the first half's MFMAs (and its code
+          // words enter each stage through fresh pinned copies): so scheduled it needs 142 VGPRs and
+          // runs three workgroups per CU (219, and two, before), and 64 rows per wave fit 256 without a
+          // spill.
+          if (FMT == 1 && hi == 0) __builtin_amdgcn_sched_barrier(0);
         }
       }
       switch (c) {
