@@ -7,8 +7,9 @@ using namespace fhip;
 
 namespace {
 
-// Up to kGemvMaxTokens tokens run the small-M GEMV kernels (decode, speculative verify); a few tens
-// q4k_mid.hip (q4k_mid_takes; small matrices from 5 tokens); more the prefill GEMM.
+// Up to kGemvMaxTokens tokens run the small-M kernels (decode, speculative verify: q4k_gemv); a few tens
+// q4k_mid.hip (q4k_mid_takes; 128 on small matrices) or, on rows too long for it, q4k_gemv16.hip; more
+// the prefill GEMM.
 constexpr int kGemvMaxTokens = 16;
 
 int check_matmul(const char *who, const void *dPacked, const float *dX, const float *dY, int out,
@@ -30,19 +31,17 @@ namespace fhip {
 int q4k_matmul_run(const void *dPacked, const float *dX, float *dY, int out, int in, int P) {
   if (P <= kGemvMaxTokens) return q4k_gemv(dPacked, dX, dY, out, in, P);
   if (q4k_mid_takes(out, in, P)) return q4k_mid(dPacked, dX, dY, out, in, P);
+  if (P <= 32) return q4k_gemv16(dPacked, dX, dY, out, in, P);
   return q4k_gemm32(dPacked, dX, dY, out, in, P);
 }
 
 size_t q4k_matmul_ws_bytes(int out, int in, int P) {
   if (P <= 0) return 0;
   if (P <= kGemvMaxTokens) return q4k_gemv_ws_bytes(out, in, P);
-  if (q4k_mid_takes(out, in, P)) {
-    // The no-allocation entry's documented bound for 17..32 tokens where that is more: what it refuses
-    // does not depend on the kernel.
-    const size_t b = q4k_mid_ws_bytes(out, in, P), doc = P <= 32 ? gemv16_ws_bytes(0, out, in, P) : 0;
-    return b > doc ? b : doc;
-  }
-  return gemm32_ws_bytes(0, out, in, P);
+  // At least the no-allocation entry's documented bound for the width, so that what it refuses does not
+  // depend on the kernel.
+  const size_t doc = P <= 32 ? gemv16_ws_bytes(0, out, in, P) : gemm32_ws_bytes(0, out, in, P);
+  return q4k_mid_takes(out, in, P) ? max(mid_ws_bytes(0, out, in, P), doc) : doc;
 }
 }  // namespace fhip
 

@@ -35,12 +35,10 @@ struct GemvGroup {
   int count;
 };
 int q4k_gemv_group(const GemvGroup &g, const float *X, int K, int M);
-// 5..16 tokens (3..16 for K >= 24576) on the 32x32x16 MFMA with exact weight operands (q4k_gemv16.hip).
+// Up to 32 tokens on the 32x32x16 MFMA with exact weight operands, sixteen at a time (q4k_gemv16.hip).
 int q4k_gemv16(const void *W, const float *X, float *Y, int N, int K, int M);
-// Scratch bytes of a q4k_gemv16 (fmt 0) / q6k_gemv16 or q6k_gemv32 (fmt 1) call.
+// Scratch bytes of a q4k_gemv16 (fmt 0) / q6k_gemv16 (fmt 1) call.
 size_t gemv16_ws_bytes(int fmt, int N, int K, int M);
-// 17..32 tokens of a Q6_K weight on the same kernel with one f16 operand row per token.
-int q6k_gemv32(const void *W, const float *X, float *Y, int N, int K, int M);
 // The same for a tiled Q6_K weight.
 int q6k_gemv16(const void *W, const float *X, float *Y, int N, int K, int M);
 // Fused decode MLP pieces (1..4 tokens): the workspace a small-M call over `ntiles` tiles
@@ -56,8 +54,10 @@ size_t q6k_gemv_ws_bytes(int N, int K, int M);
 // A few tokens to a few tens on LDS-staged operands made once per call (q4k_mid.hip): whether a call
 // takes it, its scratch bytes, the call.
 bool q4k_mid_takes(int N, int K, int M);
-size_t q4k_mid_ws_bytes(int N, int K, int M);
+bool q6k_mid_takes(int N, int K, int M);
+size_t mid_ws_bytes(int fmt, int N, int K, int M);
 int q4k_mid(const void *W, const float *X, float *Y, int N, int K, int M);
+int q6k_mid(const void *W, const float *X, float *Y, int N, int K, int M);
 int q4k_gemm32(const void *W, const float *X, float *Y, int N, int K, int M);
 // Scratch bytes of a q4k_gemm32 (fmt 0) / q6k_gemm32 (fmt 1) call.
 size_t gemm32_ws_bytes(int fmt, int N, int K, int M);

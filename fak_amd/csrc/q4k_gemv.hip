@@ -890,13 +890,13 @@ void q4k_gemv1_shape(int ntiles, int K, int &TW, int &KW) {
 
 // Scratch bytes of a 1..16-token Q4_K matmul of an [N, K] weight (the route q4k_gemv takes).
 size_t q4k_gemv_ws_bytes(int N, int K, int M) {
-  if (q4k_mid_takes(N, K, M)) return max(q4k_mid_ws_bytes(N, K, M), gemv16_ws_bytes(0, N, K, M));
+  if (q4k_mid_takes(N, K, M)) return max(mid_ws_bytes(0, N, K, M), gemv16_ws_bytes(0, N, K, M));
   if (M >= gemv16_from(K)) return gemv16_ws_bytes(0, N, K, M);
   return gemv_i8_ws_bytes(q4k_tiles(N), K, M, false);
 }
 
 // Small-M entry: 1..4 tokens on the int8 kernel, 5..16 (3..16 for K >= 24576) on the 32x32 MFMA
-// kernels of q4k_mid.hip (small matrices) and q4k_gemv16.hip.
+// kernels of q4k_mid.hip (q4k_mid_takes) and q4k_gemv16.hip.
 int q4k_gemv(const void *Wv, const float *X, float *Y, int N, int K, int M) {
   if (M < 1 || M > 16) return fail(FHIP_EINVAL, "q4k_gemv: M=%d outside 1..16", M);
   if (q4k_mid_takes(N, K, M)) return q4k_mid(Wv, X, Y, N, K, M);

@@ -1,22 +1,27 @@
-// q4k_mid.hip — Q4_K matmul for a few tokens to a few tens (speculative verify on small matrices,
-// short prompts) on the 32x32x16 f16 MFMA.
+// q4k_mid.hip — Q4_K and Q6_K matmul for a few tokens to a few tens (speculative verify, short prompts;
+// up to 128 on small matrices) on the 32x32x16 f16 MFMA.
 //
-// The arithmetic is that of q4k_gemv16.hip: weight operands are the exact integers sc_s * n, each
-// super-block's f32 result is scaled by the row's d, the min term is one more MFMA over the sub-block
-// sums, and activations are scaled by a power of two per (token, K range) that puts the range's
-// largest magnitude in [2^13, 2^14). Up to 16 tokens the 32 operand rows are the f16 of each value and
-// the f16 of its remainder (~22 bits); above, 32 tokens in f16.
+// The arithmetic is that of q4k_gemv16.hip: weight operands are exact (Q4_K the integers sc_s * n, Q6_K
+// sc_g (q - 32) / 4 as two operands), each super-block's f32 result is scaled by the row's d, Q4_K's min
+// term is one more MFMA over the sub-block sums, and activations are scaled by a power of two per
+// (token, K range) that puts the range's largest magnitude in [2^13, 2^14). Up to 16 tokens the 32
+// operand rows are the f16 of each value and the f16 of its remainder (~22 bits); above, 32 tokens in
+// f16.
 //
 // The data path is another: the operands are made once per call (mid_xprep_kernel), not by every
 // workgroup, and every workgroup streams them and its weight records to LDS by direct loads two
 // stages ahead, so no load returns to a register and nothing but the MFMAs' own operands is converted
-// in the loop. What bounds it: a workgroup's super-block takes about 1.15 us (its 37 KB through the
-// direct loads, and a wave's own chain of unpack and MFMA), so time is the longest range, plus the
-// launches before and after it. us per call against the kernels it replaced (q4k_gemv16.hip up to 16
-// tokens and its 32-token form up to 32, the prefill GEMM for more): 4096 x 4096 at 5 / 16 / 32 / 64 /
-// 128 tokens 14.3 / 14.7 / 14.8 / 22.1 / 23.8 -> 11.4 / 11.9 / 13.3 / 16.4 / 19.8; 4096 x 11008 at 32 /
-// 64 27.6 / 30.5 -> 16.7 / 24.6; 18944 x 3584 28.6 / 31.7 -> 21.6 / 27.9; 25600 x 5120 40.2 / 46.8 ->
-// 29.8 / 38.6.
+// in the loop. What bounds it: a workgroup's super-block takes about 1.15 us (Q6_K 1.6: a wave's own
+// chain of LDS reads, unpack and MFMAs; its 37 (44) KB of direct loads hide behind it), two on a CU
+// 1.7 (2.5), near the memory's pace; so time is the longest range, plus the launches before and after it.
+// us per call against the kernels it replaced (q4k_gemv16.hip, up to 16 tokens and its former 32-token
+// form up to 32, the prefill GEMM for more):
+//   Q4_K 3584 x 3584 at 8 / 16 / 32 / 64 tokens   18.1 / 18.6 / 18.2 / 22.8 -> 10.7 / 11.4 / 12.7 / 15.1
+//        18944 x 3584                             19.3 / 20.7 / 29.0 / 31.3 -> 17.7 / 18.6 / 20.1 / 25.9
+//        8192 x 11008                             28.0 / 29.5 / 39.3 / 37.3 -> 19.3 / 21.5 / 21.9 / 29.0
+//   Q6_K 3584 x 3584 at 2 / 16 / 32 / 64          18.2 / 18.8 / 21.5 / 23.2 -> 11.6 / 13.1 / 14.1 / 17.1
+//        18944 x 3584                             26.1 / 28.0 / 34.7 / 35.3 -> 21.2 / 23.0 / 24.5 / 32.0
+//        5120 x 25600                             41.8 / 45.6 / 55.2 / 58.2 -> 35.7 / 37.8 / 39.2 / 50.6
 #include <type_traits>
 
 #include "kernels.hpp"
@@ -136,42 +141,54 @@ constexpr int wait_vm_mid(int n) { return 0x0070 | (n & 15) | ((n >> 4) << 14); 
 // Workgroup = NW waves x 32 rows x TT operand tiles over one K range. A stage is half a super-block:
 // 8 operand units per tile, shared by the waves, and each wave's two record parts; three buffers, each
 // stage loaded two ahead. The super-block's headers and sum units come with its first half.
-template <int TT, bool HL, int NW>
-__global__ __launch_bounds__(64 * NW) void q4k_mid_kernel(const uint8_t *__restrict__ W,
-                                                          const u32x4 *__restrict__ xa,
-                                                          const float *__restrict__ tscale,
-                                                          float *__restrict__ Y, float *__restrict__ part,
-                                                          int N, int M, int nblk, int ntiles, int MTG,
-                                                          int tokens, int SK) {
-  constexpr int kAU = TT * 8 * 64, kWW = 2 * 64;  // operand units of a stage; a wave's record units
+template <int FMT, int TT, bool HL, int NW>  // FMT 0: Q4_K, 1: Q6_K
+__global__ __launch_bounds__(64 * NW) void quant_mid_kernel(const uint8_t *__restrict__ W,
+                                                            const u32x4 *__restrict__ xa,
+                                                            const float *__restrict__ tscale,
+                                                            float *__restrict__ Y, float *__restrict__ part,
+                                                            int N, int M, int nblk, int ntiles, int MTG,
+                                                            int tokens, int SK) {
+  constexpr int kRec = FMT == 0 ? kQ4kRecord : kQ6kRecord, kWL = FMT == 0 ? 2 : 3;  // record loads per stage
+  constexpr int kAU = TT * 8 * 64, kWW = kWL * 64;  // operand units of a stage; a wave's record units
   constexpr int kSU = kAU + NW * kWW;             // one stage: operands, then each wave's records
-  constexpr int kHU = NW * 64 + TT * 64;          // per super-block: headers (32 + 32 repeats), S units
+  constexpr int kHU = NW * 64 + (FMT == 0 ? TT * 64 : 0);  // per super-block: headers, Q4_K S units
   __shared__ u32x4 S0[kSU], S1[kSU], S2[kSU];
   __shared__ u32x4 H0[kHU], H1[kHU], H2[kHU];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kap = lane >> 5, rho = lane & 31, r16 = rho & 15;
-  const int sp = blockIdx.x % SK, task = blockIdx.x / SK, mg = task % MTG, ng = task / MTG;
+  // Workgroups go to the 8 XCDs in turn; each XCD takes a contiguous run of (range, rows, tokens), so its
+  // L2 holds the operands of one or two ranges and a record read for one token group serves the next.
+  const int x = blockIdx.x & 7, per = gridDim.x >> 3, id = x * per + min(x, (int)(gridDim.x & 7)) + (blockIdx.x >> 3);
+  const int tasks = gridDim.x / SK, sp = id / tasks, task = id - sp * tasks, mg = task % MTG, ng = task / MTG;
   const int b0 = sp * nblk / SK, b1 = (sp + 1) * nblk / SK, nb = b1 - b0;
   const int tile0 = 2 * NW * ng + 2 * wave;
   const int t0c = min(tile0, ntiles - 1), t1c = min(tile0 + 1, ntiles - 1);
   auto sbuf = [&](int k) -> u32x4 * { return k == 0 ? S0 : k == 1 ? S1 : S2; };
   auto hbuf = [&](int k) -> u32x4 * { return k == 0 ? H0 : k == 1 ? H1 : H2; };
   const int off16 = 16 * lane;
-  const int offh = (lane & 16 ? (t1c - t0c) * nblk * kQ4kRecord : 0) + 16 * (lane & 15);
+  // Header loads of the 32 rows (tiles t0c, t1c): Q4_K lane l row l % 32's 16 bytes; Q6_K lane l < 32 the
+  // row's scales, lanes 32..35 the rows' d, the rest repeat them.
+  const int dt = (t1c - t0c) * nblk * kRec;
+  const int offh = FMT == 0 || lane < 32 ? (lane & 16 ? dt : 0) + 16 * (lane & 15)
+                                         : (lane & 2 ? dt : 0) + kQ6kD + 16 * (lane & 1);
+  const int offq = (lane & 32 ? dt : 0) + 16 * (lane & 31);  // Q6_K: both tiles' qh
   const void *ra = xa + (size_t)TT * mg * nblk * (kSbUnits * 64);
-  const void *rw0 = W + (size_t)t0c * nblk * kQ4kRecord;
-  const void *rw1 = W + (size_t)t1c * nblk * kQ4kRecord;
+  const void *rw0 = W + (size_t)t0c * nblk * kRec;
+  const void *rw1 = W + (size_t)t1c * nblk * kRec;
   constexpr int kAL = 8 * TT / NW;  // operand loads per wave and stage
   // Stage s: half hh = s & 1 of super-block s / 2 of the range.
   auto load = [&](int b, int hh, u32x4 *sd, u32x4 *hd) {
-    const int bc = b0 + min(b, nb - 1), so = bc * kQ4kRecord;
+    const int bc = b0 + min(b, nb - 1), so = bc * kRec;
     if (hh == 0) {
       lds_load16(rw0, hd + wave * 64, offh, so);
-      lds_load16(ra, hd + (NW * 64 + (wave % TT) * 64), off16, (((wave % TT) * nblk + bc) * kSbUnits + 16) * 1024);
+      if (FMT == 0)
+        lds_load16(ra, hd + (NW * 64 + (wave % TT) * 64), off16, (((wave % TT) * nblk + bc) * kSbUnits + 16) * 1024);
     }
-    lds_load16(rw0, sd + (kAU + wave * kWW), off16, so + kQ4kHdr + 1024 * hh);
-    lds_load16(rw1, sd + (kAU + wave * kWW + 64), off16, so + kQ4kHdr + 1024 * hh);
+    constexpr int kQ = FMT == 0 ? kQ4kHdr : kQ6kQl;
+    lds_load16(rw0, sd + (kAU + wave * kWW), off16, so + kQ + 1024 * hh);
+    lds_load16(rw1, sd + (kAU + wave * kWW + 64), off16, so + kQ + 1024 * hh);
+    if (FMT == 1) lds_load16(rw0, sd + (kAU + wave * kWW + 128), offq, so + kQ6kQh + 512 * hh);
 #pragma unroll
     for (int j = 0; j < kAL; ++j) {
       const int un = kAL * wave + j, i = un >> 3, q = un & 7;  // token tile, slice of the half
@@ -193,7 +210,16 @@ __global__ __launch_bounds__(64 * NW) void q4k_mid_kernel(const uint8_t *__restr
   const uint32_t kMagic = in_reg(0x64006400u), kB02 = in_reg(0x00FF00FFu);
   const h2 k1024 = {(_Float16)1024.f, (_Float16)1024.f}, kN1024 = -k1024;
   const h2 k16th = {(_Float16)0.0625f, (_Float16)0.0625f}, k32 = {(_Float16)32.f, (_Float16)32.f};
-  constexpr int kEven = 4 + kAL, kOdd = 2 + kAL;  // loads of an even / odd stage
+  constexpr int kEven = (FMT == 0 ? 2 : 1) + kWL + kAL, kOdd = kWL + kAL;  // loads of an even / odd stage
+  // Q6_K: this lane's 8 ql bytes of (tile, group h), qh bytes and d, in units of 8 and 2 bytes.
+  const uint32_t ql = FMT == 1 ? in_reg(2 * (kAU + wave * kWW + 64 * (rho >> 4) + r16) + kap) : 0u;
+  const uint32_t qq = FMT == 1 ? in_reg(2 * (kAU + wave * kWW + 128 + 32 * (rho >> 4) + r16) + kap) : 0u;
+  const uint32_t dl = FMT == 1 ? in_reg(8 * (wave * 64 + 32 + 2 * (rho >> 4)) + r16) : 0u;
+  const uint32_t k80 = FMT == 1 ? in_reg(0x80808080u) : 0u;
+  const uint32_t kB6 = FMT == 1 ? in_reg(0x00C000C0u) : 0u, kB8 = FMT == 1 ? in_reg(0x03000300u) : 0u;
+  const h2 k1152 = {(_Float16)1152.f, (_Float16)1152.f}, k4th = {(_Float16)0.25f, (_Float16)0.25f};
+  const h2 k64th = k16th * k4th, kTb = {(_Float16)0.0625f, (_Float16)0.015625f};  // b under 2^6, 2^8
+  const h2 kOb = {(_Float16)-72.f, (_Float16)-24.f};  // -(1024 + 2 2^6) / 16, -(1024 + 2 2^8) / 64
   for (int bb = 0; bb < nb; bb += 3) {
 #pragma unroll
     for (int u = 0; u < 6; ++u) {
@@ -201,64 +227,115 @@ __global__ __launch_bounds__(64 * NW) void q4k_mid_kernel(const uint8_t *__restr
       load(b + 1, hh, sbuf((u + 2) % 3), hbuf((u / 2 + 1) % 3));
       if (b < nb) {
         const u32x4 *Sb = sbuf(u % 3), *Hb = hbuf(u / 2);
-        // the super-block's scales (read again at each half: cheaper than held registers)
-        const u32x4 hd = Hb[hl];
-        const uint32_t sc4 = hh == 0 ? hd[1] & 0x3F3F3F3Fu : (hd[3] & 0x0F0F0F0Fu) | ((hd[1] >> 2) & 0x30303030u);
-        const h2 ep = as_h2((sc4 & kB02) | kMagic) - k1024;         // sub-blocks 4 hh, 4 hh + 2
-        const h2 op = as_h2(((sc4 >> 8) & kB02) | kMagic) - k1024;  // 4 hh + 1, 4 hh + 3
-        const u32x4 nb0 = Sb[wl], nb1 = Sb[wl + 32];
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-          const _Float16 sa = c ? ep.y : ep.x, sb = c ? op.y : op.x;
-          const h2 SL = {sa, sa}, SH = h2{sb, sb} * k16th;
-          const h2 NL = SL * kN1024, NH = SH * kN1024;
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            const u32x4 q = h ? nb1 : nb0;
-            const uint32_t x0 = c ? q[2] : q[0], x1 = c ? q[3] : q[1];
-            const uint32_t y0 = x0 >> 8, y1 = x1 >> 8;
-            u32x4 lw, hw;
-            lw[0] = as_u(__builtin_elementwise_fma(as_h2((x0 & kLo) | kMagic), SL, NL));
-            lw[1] = as_u(__builtin_elementwise_fma(as_h2((y0 & kLo) | kMagic), SL, NL));
-            lw[2] = as_u(__builtin_elementwise_fma(as_h2((x1 & kLo) | kMagic), SL, NL));
-            lw[3] = as_u(__builtin_elementwise_fma(as_h2((y1 & kLo) | kMagic), SL, NL));
-            hw[0] = as_u(__builtin_elementwise_fma(as_h2((x0 & kHi) | kMagic), SH, NH));
-            hw[1] = as_u(__builtin_elementwise_fma(as_h2((y0 & kHi) | kMagic), SH, NH));
-            hw[2] = as_u(__builtin_elementwise_fma(as_h2((x1 & kHi) | kMagic), SH, NH));
-            hw[3] = as_u(__builtin_elementwise_fma(as_h2((y1 & kHi) | kMagic), SH, NH));
-#pragma unroll
-            for (int hi = 0; hi < 2; ++hi)
-#pragma unroll
-              for (int i = 0; i < TT; ++i) {
-                const f16x8 a = __builtin_bit_cast(f16x8, Sb[(i * 8 + 4 * c + 2 * hi + h) * 64 + al]);
-                f32x16 z = tmp[i][hi];
-                if (hh == 0 && c == 0 && h == 0)
-#pragma unroll
-                  for (int e = 0; e < 16; ++e) z[e] = 0.f;
-                tmp[i][hi] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, __builtin_bit_cast(f16x8, hi ? hw : lw), z, 0, 0, 0);
-              }
+        if constexpr (FMT == 0) {
+          // the super-block's scales (read again at each half: cheaper than held registers)
+          const u32x4 hd = Hb[hl];
+          const uint32_t sc4 = hh == 0 ? hd[1] & 0x3F3F3F3Fu : (hd[3] & 0x0F0F0F0Fu) | ((hd[1] >> 2) & 0x30303030u);
+          const h2 ep = as_h2((sc4 & kB02) | kMagic) - k1024;         // sub-blocks 4 hh, 4 hh + 2
+          const h2 op = as_h2(((sc4 >> 8) & kB02) | kMagic) - k1024;  // 4 hh + 1, 4 hh + 3
+          const u32x4 nb0 = Sb[wl], nb1 = Sb[wl + 32];
+  #pragma unroll
+          for (int c = 0; c < 2; ++c) {
+            const _Float16 sa = c ? ep.y : ep.x, sb = c ? op.y : op.x;
+            const h2 SL = {sa, sa}, SH = h2{sb, sb} * k16th;
+            const h2 NL = SL * kN1024, NH = SH * kN1024;
+  #pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const u32x4 q = h ? nb1 : nb0;
+              const uint32_t x0 = c ? q[2] : q[0], x1 = c ? q[3] : q[1];
+              const uint32_t y0 = x0 >> 8, y1 = x1 >> 8;
+              u32x4 lw, hw;
+              lw[0] = as_u(__builtin_elementwise_fma(as_h2((x0 & kLo) | kMagic), SL, NL));
+              lw[1] = as_u(__builtin_elementwise_fma(as_h2((y0 & kLo) | kMagic), SL, NL));
+              lw[2] = as_u(__builtin_elementwise_fma(as_h2((x1 & kLo) | kMagic), SL, NL));
+              lw[3] = as_u(__builtin_elementwise_fma(as_h2((y1 & kLo) | kMagic), SL, NL));
+              hw[0] = as_u(__builtin_elementwise_fma(as_h2((x0 & kHi) | kMagic), SH, NH));
+              hw[1] = as_u(__builtin_elementwise_fma(as_h2((y0 & kHi) | kMagic), SH, NH));
+              hw[2] = as_u(__builtin_elementwise_fma(as_h2((x1 & kHi) | kMagic), SH, NH));
+              hw[3] = as_u(__builtin_elementwise_fma(as_h2((y1 & kHi) | kMagic), SH, NH));
+  #pragma unroll
+              for (int hi = 0; hi < 2; ++hi)
+  #pragma unroll
+                for (int i = 0; i < TT; ++i) {
+                  const f16x8 a = __builtin_bit_cast(f16x8, Sb[(i * 8 + 4 * c + 2 * hi + h) * 64 + al]);
+                  f32x16 z = tmp[i][hi];
+                  if (hh == 0 && c == 0 && h == 0)
+  #pragma unroll
+                    for (int e = 0; e < 16; ++e) z[e] = 0.f;
+                  tmp[i][hi] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, __builtin_bit_cast(f16x8, hi ? hw : lw), z, 0, 0, 0);
+                }
+            }
           }
-        }
-        if (hh == 1) {
-          const float d = (float)__builtin_bit_cast(_Float16, (uint16_t)(hd[0] & 0xffffu));
-          const float dm = (float)__builtin_bit_cast(_Float16, (uint16_t)(hd[0] >> 16));
-          const uint32_t mnl = hd[2] & 0x3F3F3F3Fu;
-          const uint32_t mnh = ((hd[3] >> 4) & 0x0F0F0F0Fu) | ((hd[2] >> 2) & 0x30303030u);
-          u32x4 mw;
-          mw[0] = as_u((as_h2((mnl & kB02) | kMagic) - k1024) * k32);
-          mw[1] = as_u((as_h2(((mnl >> 8) & kB02) | kMagic) - k1024) * k32);
-          mw[2] = as_u((as_h2((mnh & kB02) | kMagic) - k1024) * k32);
-          mw[3] = as_u((as_h2(((mnh >> 8) & kB02) | kMagic) - k1024) * k32);
+          if (hh == 1) {
+            const float d = (float)__builtin_bit_cast(_Float16, (uint16_t)(hd[0] & 0xffffu));
+            const float dm = (float)__builtin_bit_cast(_Float16, (uint16_t)(hd[0] >> 16));
+            const uint32_t mnl = hd[2] & 0x3F3F3F3Fu;
+            const uint32_t mnh = ((hd[3] >> 4) & 0x0F0F0F0Fu) | ((hd[2] >> 2) & 0x30303030u);
+            u32x4 mw;
+            mw[0] = as_u((as_h2((mnl & kB02) | kMagic) - k1024) * k32);
+            mw[1] = as_u((as_h2(((mnl >> 8) & kB02) | kMagic) - k1024) * k32);
+            mw[2] = as_u((as_h2((mnh & kB02) | kMagic) - k1024) * k32);
+            mw[3] = as_u((as_h2(((mnh >> 8) & kB02) | kMagic) - k1024) * k32);
+  #pragma unroll
+            for (int i = 0; i < TT; ++i) {
+              f32x16 mt;
+  #pragma unroll
+              for (int e = 0; e < 16; ++e) mt[e] = 0.f;
+              mt = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, Hb[(NW + i) * 64 + al]),
+                                                          __builtin_bit_cast(f16x8, mw), mt, 0, 0, 0);
+  #pragma unroll
+              for (int e = 0; e < 16; ++e)
+                acc[i][e] = fmaf(d, tmp[i][0][e] + tmp[i][1][e], fmaf(-dm, mt[e], acc[i][e]));
+            }
+          }
+        } else {
+          // Q6_K: group g = K16 slice g. With q = n + 16 b (nibble n, qh field b), sc_g (q - 32) / 4 is the
+          // sum of two operands that f16 holds exactly, sc_g n / 4 (up to 480) and 4 sc_g (b - 2) (up to
+          // 1024), each one fma of the field under the exponent of 1024 (n 2^(4 c), b 2^(6 + 2 hi)).
+          const uint2 *Q = reinterpret_cast<const uint2 *>(Sb);
+          const u32x4 hd = Hb[hl];
 #pragma unroll
-          for (int i = 0; i < TT; ++i) {
-            f32x16 mt;
+          for (int c = 0; c < 2; ++c) {
+            const uint32_t sw = hd[2 * hh + c] ^ k80;
 #pragma unroll
-            for (int e = 0; e < 16; ++e) mt[e] = 0.f;
-            mt = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, Hb[(NW + i) * 64 + al]),
-                                                        __builtin_bit_cast(f16x8, mw), mt, 0, 0, 0);
+            for (int h = 0; h < 2; ++h) {
+              const h2 P = as_h2(((h ? sw >> 8 : sw) & kB02) | kMagic) - k1152;  // scales of hi = 0, 1
+              const h2 SP = P * (c ? k64th : k4th), NP = SP * kN1024, TP = P * kTb, OP = P * kOb;
+              const uint2 qa = Q[ql + 32 * h], qb = Q[ql + 64 + 32 * h], qh = Q[qq + 32 * h];
 #pragma unroll
-            for (int e = 0; e < 16; ++e)
-              acc[i][e] = fmaf(d, tmp[i][0][e] + tmp[i][1][e], fmaf(-dm, mt[e], acc[i][e]));
+              for (int hi = 0; hi < 2; ++hi) {
+                const _Float16 s = hi ? SP.y : SP.x, n = hi ? NP.y : NP.x, t = hi ? TP.y : TP.x, o = hi ? OP.y : OP.x;
+                const h2 S = {s, s}, N0 = {n, n}, T = {t, t}, O = {o, o};
+                const uint32_t mn = c ? kHi : kLo, mb = hi ? kB8 : kB6;
+                u32x4 vn, vb;
+#pragma unroll
+                for (int m = 0; m < 2; ++m) {
+                  const uint32_t x = hi ? (m ? qb.y : qb.x) : (m ? qa.y : qa.x), b4 = m ? qh.y : qh.x;
+                  const uint32_t be = b4 << (c ? 2 : 6), bo = b4 >> (c ? 6 : 2);
+                  vn[2 * m] = as_u(__builtin_elementwise_fma(as_h2((x & mn) | kMagic), S, N0));
+                  vn[2 * m + 1] = as_u(__builtin_elementwise_fma(as_h2(((x >> 8) & mn) | kMagic), S, N0));
+                  vb[2 * m] = as_u(__builtin_elementwise_fma(as_h2((be & mb) | kMagic), T, O));
+                  vb[2 * m + 1] = as_u(__builtin_elementwise_fma(as_h2((bo & mb) | kMagic), T, O));
+                }
+#pragma unroll
+                for (int i = 0; i < TT; ++i) {
+                  const f16x8 a = __builtin_bit_cast(f16x8, Sb[(i * 8 + 4 * c + 2 * hi + h) * 64 + al]);
+                  f32x16 z = tmp[i][0], y = tmp[i][1];
+                  if (hh == 0 && c == 0 && h == 0 && hi == 0)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) z[e] = y[e] = 0.f;
+                  tmp[i][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, __builtin_bit_cast(f16x8, vn), z, 0, 0, 0);
+                  tmp[i][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, __builtin_bit_cast(f16x8, vb), y, 0, 0, 0);
+                }
+              }
+            }
+          }
+          if (hh == 1) {
+            const float d = 4.f * (float)reinterpret_cast<const _Float16 *>(Hb)[dl];
+#pragma unroll
+            for (int i = 0; i < TT; ++i)
+#pragma unroll
+              for (int e = 0; e < 16; ++e) acc[i][e] = fmaf(d, tmp[i][0][e] + tmp[i][1][e], acc[i][e]);
           }
         }
       }
@@ -299,6 +376,8 @@ __global__ __launch_bounds__(64 * NW) void q4k_mid_kernel(const uint8_t *__restr
 
 namespace {
 
+constexpr int kMidRanges = 64;  // what sum_ranges reads at once
+
 struct MidPlan {
   bool hl;
   int TT, NW, MTG, tokens, tasks, SK;
@@ -306,11 +385,17 @@ struct MidPlan {
   float cost;
 };
 
-// The K split with the lowest estimated time (us): the longest range's super-blocks at the pace of one
-// workgroup per CU (t1), or of two (t2, where two fit), in as many rounds as the grid takes, and for a
-// split the launch that adds the ranges and its traffic. Fitted to sweeps of the range count at ten
-// shapes from 1536 x 1024 to 5120 x 25600; the choice is the best or within 4% of it at each.
-MidPlan plan_mid(int N, int K, int M, int TT, int NW) {
+// The K split with the lowest estimated time (us): the super-blocks of a range (between the mean and the
+// longest) at the pace of one workgroup per CU, or of two where the grid gives a CU two and they fit, in
+// as many rounds as the grid takes, and for a split the launch that adds the ranges and its traffic.
+// Fitted to sweeps of the range count at 75 shapes from 500 x 1024 to 25600 x 5120 and 2..128 tokens:
+// the choice is within 1.5% of the best there on average, 10% at the worst.
+struct MidPace {
+  float one, two, wide, longest, start, launch, range, traffic;
+};
+constexpr MidPace kMidPace[2] = {{1.13f, 1.68f, 2.15f, 0.61f, 0.4f, 1.9f, 0.06f, 7.4f / 3.5e6f},
+                                 {1.52f, 2.53f, 3.67f, 0.87f, 1.3f, 1.9f, 0.07f, 6.0f / 3.5e6f}};
+MidPlan plan_mid(int fmt, int N, int K, int M, int TT, int NW) {
   MidPlan p{};
   const int nblk = K / 256, cus = cu_count() > 0 ? cu_count() : 256;
   p.hl = M <= 16;
@@ -319,18 +404,20 @@ MidPlan plan_mid(int N, int K, int M, int TT, int NW) {
   p.MTG = p.hl ? 1 : ceil_div(M, 32 * TT);
   p.tokens = p.hl ? 16 : 32 * TT * p.MTG;
   p.tasks = p.MTG * ceil_div(N, 32 * NW);
-  const float t1 = TT == 2 ? 2.0f : 1.15f, t2 = 1.9f;
+  const MidPace &m = kMidPace[fmt];
   const int fit = NW == 8 ? 1 : 2;  // workgroups per CU
-  for (int sk = 1; sk <= nblk && sk <= 32; ++sk) {
+  for (int sk = 1; sk <= nblk && sk <= kMidRanges; ++sk) {
     const long long wgs = (long long)p.tasks * sk;
-    const float pace = wgs <= cus || fit == 1 ? t1 : t2;
+    const float pace = fit == 1 ? m.wide : wgs <= cus ? m.one : m.two;
     const float rounds = wgs <= cus ? 1.f : (float)((wgs + fit * cus - 1) / (fit * cus));
-    const float c = rounds * ceil_div(nblk, sk) * pace +
-                    (sk > 1 ? 2.2f + 8.f * sk * (float)M * (float)N / 3.5e6f : 0.f);
+    const float len = m.longest * ceil_div(nblk, sk) + (1.f - m.longest) * nblk / sk;
+    const float c = rounds * (len * pace + m.start) +
+                    (sk > 1 ? m.launch + m.range * sk + m.traffic * sk * (float)M * (float)N : 0.f);
     if (sk == 1 || c < p.cost) {
       p.cost = c;
       p.SK = sk;
     }
+    if (rounds > 3.f) break;  // more ranges only add rounds
   }
   p.xb = (size_t)(p.hl ? 1 : TT * p.MTG) * nblk * kSbUnits * 1024;
   p.tb = ((size_t)p.SK * p.tokens * 4 + 255) & ~(size_t)255;
@@ -341,40 +428,59 @@ MidPlan plan_mid(int N, int K, int M, int TT, int NW) {
 // One operand tile and four waves per workgroup, or (above 32 tokens) two tiles and eight waves, which
 // halve the operand traffic of a large matrix: 64 tokens of 18944 x 3584 32.2 / 28.3 us, of 3584 x 3584
 // 14.8 / 18.6.
-MidPlan plan_mid(int N, int K, int M) {
-  const MidPlan p = plan_mid(N, K, M, 1, 4);
+MidPlan plan_mid(int fmt, int N, int K, int M) {
+  const MidPlan p = plan_mid(fmt, N, K, M, 1, 4);
   if (M <= 32) return p;
-  const MidPlan q = plan_mid(N, K, M, 2, 8);
+  const MidPlan q = plan_mid(fmt, N, K, M, 2, 8);
   return q.cost < p.cost ? q : p;
 }
 
 }  // namespace
 
-// Which calls take this kernel (us, before / here). Up to 16 tokens matrices of up to 36 M weights
-// (3584 x 3584 at 8 tokens 17.8 / 10.6, 8192 x 4096 14.6 / 13.4, 4096 x 8192 15.0 / 13.4; larger ones
-// mostly lose: 11008 x 4096 15.2 / 15.8, 25600 x 5120 23.9 / 27); 17..64 tokens all (8192 x 4096 at 32,
-// the closest, 17.4 / 16.1); 65..128 small matrices (4096 x 4096 at 128 tokens 24.0 / 20.7, 8192 x 4096
-// at 65 23.7 / 25.2). Rows long enough to make the operands large keep the other kernels.
+namespace {
+// Up to 16 tokens: all but few rows of more than 96 super-blocks, where the workgroups of
+// q4k_gemv16.hip already fill the chip and need no launch before them. (us, that kernel / this, 16
+// tokens: Q6_K 1000 x 25600 17.6 / 18.3, 3584 x 25600 32.8 / 26.9; 8 tokens of Q4_K 2560 x 25600 17.8 /
+// 18.4, 3584 x 25600 22.7 / 20.1.) 17..64: all. 65..128: matrices of up to w128 weights, whose prefill
+// GEMM runs too few tiles. Rows long enough to make the operands large keep the other kernels.
+bool mid_takes(int N, int K, int M, long long w128) {
+  if (K > 262144) return false;
+  if (M <= 16) return K <= 24576 || N >= 3072;
+  return M <= 64 || (M <= 128 && (long long)N * K <= w128);
+}
+}  // namespace
+
+// Besides, up to 16 tokens of Q4_K: matrices of more than 100 M weights are as fast without the operand
+// launch (25600 x 5120 at 8 tokens 23.9 / 24.2), and so are ones that q4k_gemv16.hip divides into equal
+// ranges of one workgroup per CU (11008 x 5120 15.6 / 16.4). 65..128 tokens (us, GEMM / this): 24 M
+// weights (11008 x 2048 at 128 24.1 / 21.8), on long rows 70 M, as the GEMM's ranges there are short
+// (1536 x 25600 36.8 / 32.0, 3584 x 18944 43.6 / 39.7), not on many short rows (18944 x 1024 17.7 / 18.2).
 bool q4k_mid_takes(int N, int K, int M) {
   const long long w = (long long)N * K;
-  if (M < 5 || K > 262144) return false;
-  if (M <= 16) return w <= 36000000;
-  if (M <= 64) return true;
-  return M <= 128 && w <= 20000000;
+  const int nblk = K / 256;
+  if (M < 5 || (M > 64 && N > 12288)) return false;
+  if (M <= 16 && w > 100000000) return false;
+  if (M <= 16 && w > 50000000 && nblk % 4 == 0 && (long long)ceil_div(N, 256) * (nblk / 4) <= cu_count()) return false;
+  return mid_takes(N, K, M, K > 10240 ? 70000000 : 24000000);
 }
 
-size_t q4k_mid_ws_bytes(int N, int K, int M) {
-  const MidPlan p = plan_mid(N, K, M);
+// 65..128 tokens: 8192 x 2048 at 128 25.8 / 20.6, 1536 x 8192 20.8 / 17.9.
+bool q6k_mid_takes(int N, int K, int M) { return M >= 2 && mid_takes(N, K, M, 1 << 24); }
+
+size_t mid_ws_bytes(int fmt, int N, int K, int M) {
+  const MidPlan p = plan_mid(fmt, N, K, M);
   return p.xb + p.tb + p.pb;
 }
 
-int q4k_mid(const void *Wv, const float *X, float *Y, int N, int K, int M) {
-  const MidPlan p = plan_mid(N, K, M);
+namespace {
+template <int FMT>
+int launch_mid(const void *Wv, const float *X, float *Y, int N, int K, int M) {
+  const MidPlan p = plan_mid(FMT, N, K, M);
   const int nblk = K / 256, ntiles = q4k_tiles(N), SK = p.SK, MTG = p.MTG, tokens = p.tokens;
   const size_t xb = p.xb, tb = p.tb, pb = p.pb;
   unsigned char *ws = (unsigned char *)workspace(xb + tb + pb);
   if (!ws) return FHIP_ENOMEM;
-  if (int rc = check_disjoint("q4k_mid", X, (size_t)M * K * 4, ws, xb + tb + pb)) return rc;
+  if (int rc = check_disjoint("quant_mid", X, (size_t)M * K * 4, ws, xb + tb + pb)) return rc;
   u32x4 *xa = (u32x4 *)ws;
   float *ts = (float *)(ws + xb), *part = (float *)(ws + xb + tb);
   const dim3 pg(tokens, SK);
@@ -398,13 +504,22 @@ int q4k_mid(const void *Wv, const float *X, float *Y, int N, int K, int M) {
     kern<<<p.tasks * SK, 64 * p.NW, 0, stream()>>>(W, xa, ts, Y, part, N, M, nblk, ntiles, MTG, tokens, SK);
   };
   if (p.hl)
-    run(q4k_mid_kernel<1, true, 4>);
+    run(quant_mid_kernel<FMT, 1, true, 4>);
   else if (p.TT == 1)
-    run(q4k_mid_kernel<1, false, 4>);
+    run(quant_mid_kernel<FMT, 1, false, 4>);
   else
-    run(q4k_mid_kernel<2, false, 8>);
-  FHIP_CHECK_LAUNCH("q4k_mid_kernel");
+    run(quant_mid_kernel<FMT, 2, false, 8>);
+  FHIP_CHECK_LAUNCH("quant_mid_kernel");
   return SK > 1 ? sum_ranges(part, Y, SK, M * N) : FHIP_OK;
+}
+}  // namespace
+
+int q4k_mid(const void *W, const float *X, float *Y, int N, int K, int M) {
+  return launch_mid<0>(W, X, Y, N, K, M);
+}
+
+int q6k_mid(const void *W, const float *X, float *Y, int N, int K, int M) {
+  return launch_mid<1>(W, X, Y, N, K, M);
 }
 
 }  // namespace fhip

@@ -164,10 +164,11 @@ int fhip_q4k_matmul_int8_f32(const void *dPacked, const float *dX, float *dY, in
  * their scratch (activation operands, token scales, K-range partial sums) in a static 64 MiB
  * device array per device instead of the library workspace, and calls no hipMalloc / hipFree.
  * A call whose scratch would exceed 64 MiB returns FHIP_EINVAL without launching anything.
- * The scratch is: for 1..4 tokens at most in/256 * 3.3 KB; for 5..32 tokens (3..32 when
- * in >= 24576) the K-range partial sums, 4 * P * out bytes per 1,024 values of in (about
- * in * out * P / 256 bytes); for the prefill GEMM its f16 operands (2 * P * in bytes) plus
- * partial sums when K is split. So every 7B / 27B FFN, attention and 152064 x 3584 lm_head
+ * The scratch counted is: for 1..4 tokens at most in/256 * 3.3 KB; for 5..32 tokens (3..32
+ * when in >= 24576) the larger of 4 * P * out bytes per 1,024 values of in (about in * out * P /
+ * 256 bytes) and, where the kernel for a few tens of tokens runs, its f16 operands (17 KB per 256
+ * values of in) plus K-range partial sums; for more, the larger of the prefill GEMM's f16 operands
+ * (2 * P * in bytes, P in whole 128s) plus partial sums when K is split, and that kernel's. So every 7B / 27B FFN, attention and 152064 x 3584 lm_head
  * call of up to 32 tokens fits, and so does a prefill of 512 tokens at the 7B shapes; a
  * 16-token call on a 17408 x 65536 weight (71 MB) and a 1,024-token prefill through the
  * 18944 -> 3584 projection do not. The array keeps the last call's contents and is shared by
