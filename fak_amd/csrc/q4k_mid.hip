@@ -291,7 +291,9 @@ __global__ __launch_bounds__(64 * NW) void quant_mid_kernel(const uint8_t *__res
         } else {
           // Q6_K: group g = K16 slice g. With q = n + 16 b (nibble n, qh field b), sc_g (q - 32) / 4 is the
           // sum of two operands that f16 holds exactly, sc_g n / 4 (up to 480) and 4 sc_g (b - 2) (up to
-          // 1024), each one fma of the field under the exponent of 1024 (n 2^(4 c), b 2^(6 + 2 hi)).
+          // 1024), each one fma of the field under the exponent of 1024 (n 2^(4 c), b 2^(6 + 2 hi)). Both
+          // feed one chain, whose running sum is that of the whole weights: with a chain each the error
+          // against 64 bits is 4% larger.
           const uint2 *Q = reinterpret_cast<const uint2 *>(Sb);
           const u32x4 hd = Hb[hl];
 #pragma unroll
@@ -320,12 +322,12 @@ __global__ __launch_bounds__(64 * NW) void quant_mid_kernel(const uint8_t *__res
 #pragma unroll
                 for (int i = 0; i < TT; ++i) {
                   const f16x8 a = __builtin_bit_cast(f16x8, Sb[(i * 8 + 4 * c + 2 * hi + h) * 64 + al]);
-                  f32x16 z = tmp[i][0], y = tmp[i][1];
-                  if (hh == 0 && c == 0 && h == 0 && hi == 0)
+                  f32x16 z = tmp[i][hi];
+                  if (hh == 0 && c == 0 && h == 0)
 #pragma unroll
-                    for (int e = 0; e < 16; ++e) z[e] = y[e] = 0.f;
-                  tmp[i][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, __builtin_bit_cast(f16x8, vn), z, 0, 0, 0);
-                  tmp[i][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, __builtin_bit_cast(f16x8, vb), y, 0, 0, 0);
+                    for (int e = 0; e < 16; ++e) z[e] = 0.f;
+                  z = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, __builtin_bit_cast(f16x8, vn), z, 0, 0, 0);
+                  tmp[i][hi] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, __builtin_bit_cast(f16x8, vb), z, 0, 0, 0);
                 }
               }
             }
