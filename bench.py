@@ -169,8 +169,8 @@ def spread_sample(raw, n, k, per_block=2, block=128):
 
 def bench_crossover(steps, warmup, ev, tokens=(1, 2, 4, 8, 16, 17, 24, 32, 48, 64, 128)):
     """The small-M -> MFMA crossover on the C3 shape (K=3584 -> N=18944): every route
-    fhip_q4k_matmul_f32 takes by token count (int8 GEMV 1..4, the 32x32 hi/lo GEMV 5..16, its
-    f16 form 17..32, the prefill GEMM beyond), back to back over the rotating weight copies."""
+    fhip_q4k_matmul_f32 takes by token count (int8 GEMV 1..4, the staged 32x32 kernel
+    with hi/lo operands 5..16 and f16 ones 17..64, the prefill GEMM beyond), back to back over the rotating weight copies."""
     n, k = 18944, 3584
     w = Weight("q4k", n, k, 3, copies_for(q4k_bytes(n, k)))
     out = []
@@ -180,8 +180,8 @@ def bench_crossover(steps, warmup, ev, tokens=(1, 2, 4, 8, 16, 17, 24, 32, 48, 6
         ms, _ = time_calls([("fhip_q4k_matmul_f32",
                              lambda i: (w.ptrs[i % len(w.ptrs)], xb.ptr, yb.ptr, n, k, M))],
                            steps, warmup, ev)
-        route = ("int8 GEMV" if M <= 4 else "32x32 GEMV, hi/lo f16" if M <= 16 else
-                 "32x32 GEMV, f16" if M <= 32 else "prefill GEMM")
+        route = ("int8 GEMV" if M <= 4 else "32x32 staged, hi/lo f16" if M <= 16 else
+                 "32x32 staged, f16" if M <= 64 else "prefill GEMM")
         out.append({"M": M, "route": route, "us_back_to_back": 1e3 * ms,
                     "GBs": q4k_bytes(n, k) / (ms * 1e6),
                     "TFLOPs": 2.0 * M * n * k / (ms * 1e-3) / 1e12})
