@@ -379,6 +379,9 @@ __global__ __launch_bounds__(64 * NW) void quant_mid_kernel(const uint8_t *__res
 namespace {
 
 constexpr int kMidRanges = 64;  // what sum_ranges reads at once
+// Operands (at most 36 MB, by mid_takes) and partial results together stay well inside the 64 MiB of the
+// no-allocation entry, whatever the shape.
+constexpr size_t kMidScratch = (size_t)48 << 20;
 
 struct MidPlan {
   bool hl;
@@ -408,7 +411,9 @@ MidPlan plan_mid(int fmt, int N, int K, int M, int TT, int NW) {
   p.tasks = p.MTG * ceil_div(N, 32 * NW);
   const MidPace &m = kMidPace[fmt];
   const int fit = NW == 8 ? 1 : 2;  // workgroups per CU
+  p.xb = (size_t)(p.hl ? 1 : TT * p.MTG) * nblk * kSbUnits * 1024;
   for (int sk = 1; sk <= nblk && sk <= kMidRanges; ++sk) {
+    if (sk > 1 && p.xb + (size_t)sk * M * N * 4 > kMidScratch) break;
     const long long wgs = (long long)p.tasks * sk;
     const float pace = fit == 1 ? m.wide : wgs <= cus ? m.one : m.two;
     const float rounds = wgs <= cus ? 1.f : (float)((wgs + fit * cus - 1) / (fit * cus));
@@ -421,7 +426,6 @@ MidPlan plan_mid(int fmt, int N, int K, int M, int TT, int NW) {
     }
     if (rounds > 3.f) break;  // more ranges only add rounds
   }
-  p.xb = (size_t)(p.hl ? 1 : TT * p.MTG) * nblk * kSbUnits * 1024;
   p.tb = ((size_t)p.SK * p.tokens * 4 + 255) & ~(size_t)255;
   p.pb = p.SK > 1 ? (size_t)p.SK * M * N * 4 : 0;
   return p;
@@ -448,7 +452,7 @@ namespace {
 bool mid_takes(int N, int K, int M, long long w128) {
   if (K > 262144) return false;
   if (M <= 16) return K <= 24576 || N >= 3072;
-  return M <= 64 || (M <= 128 && (long long)N * K <= w128);
+  return M <= 64 || (M <= 128 && K <= 131072 && (long long)N * K <= w128);
 }
 }  // namespace
 

@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 from fak_amd import synth
-from tests.gpu_util import q4k_matmul, q4k_matmul_group, rel_err_rows, scaled_activations
+from tests.gpu_util import Dev, q4k_matmul, q4k_matmul_group, rel_err_rows, scaled_activations
 
 pytestmark = pytest.mark.gpu
 
@@ -69,3 +69,21 @@ def test_group_members(hip):
     X = synth.activations(P, in_, 1)
     for raw, o, y in zip(raws, outs, q4k_matmul_group(raws, outs, in_, X, P)):
         assert rel_err_rows(y, exact(raw, o, in_, X)) <= 1e-5
+
+
+@pytest.mark.parametrize("out,in_,P", [(78848, 2560, 64), (2048, 65536, 64), (40, 262144, 32)])
+def test_scratch_stays_small(hip, out, in_, P):
+    """Operands and partial results fit the no-allocation entry's 64 MiB at tall and at long weights."""
+    lib = hip.load()
+    print(f"[case] q4k mid scratch out={out} in={in_} P={P}", flush=True)
+    raw = synth.q4k_weights(out, in_, seed=1)
+    w = hip.alloc_call("fhip_q4k_upload", np.ascontiguousarray(raw).ctypes.data, out, in_)
+    try:
+        X = synth.activations(P, in_, 1)
+        with Dev.from_host(X) as dx, Dev(P * out * 4) as dy:
+            hip.call("fhip_q4k_matmul_noalloc_f32", w, dx.ptr, dy.ptr, out, in_, P)
+            Y = dy.to_host(np.float32).reshape(P, out)
+            hip.call("fhip_q4k_matmul_f32", w, dx.ptr, dy.ptr, out, in_, P)
+            np.testing.assert_array_equal(Y, dy.to_host(np.float32).reshape(P, out))
+    finally:
+        lib.fhip_free(w)
