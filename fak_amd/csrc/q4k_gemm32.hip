@@ -945,11 +945,12 @@ GemmPlan plan_gemm32(int fmt, int N, int K, int M) {
   // 25600 x 5120 86.6 / 81.9, 896 of 3584 x 18944 179 / 171; 512 of 18944 x 3584 (592 tiles) 82.6 /
   // 84.5, of 25600 x 5120 (800) 145.8 / 147.9. Q6_K, whose records take 14 loads, is no faster so
   // (512 tokens of 18944 x 3584 94.0 / 99.3).
-  // Nor are short ranges of two and more token tiles, or of rows of up to 16 super-blocks (us, 256 tokens
-  // of 1536 x 25600 46.8 / 52.8, of 5120 x 5120 32.6 / 33.5, of 3584 x 18944 58.3 / 59.1; 100 tokens of
-  // 18944 x 3584 36.0 / 36.6; one tile of longer rows, 128 tokens: 5120 x 5120 26.7 / 24.5, 3584 x 18944
-  // 41.3 / 40.0).
-  p.deep = fmt == 0 && p.tasks < 2 * cus && ((p.MTG == 1 && nblk > 16) || p.F > 0 || nblk / p.S >= 12);
+  // Of grids split into short ranges it is the form where a CU gets one workgroup, with nothing beside it to
+  // hide a wait (us, 350 tokens of 517 x 6656 31.6 / 28.4, 128 of 5120 x 5120 26.7 / 24.5), and for one token
+  // tile of long rows (128 tokens of 3584 x 18944 41.3 / 40.0); not for more of either (256 tokens of
+  // 1536 x 25600 46.8 / 52.8, of 5120 x 5120 32.6 / 33.5; 100 tokens of 18944 x 3584 36.0 / 36.6).
+  p.deep = fmt == 0 && p.tasks < 2 * cus &&
+           (p.F > 0 || p.R * p.S <= cus || (p.MTG == 1 && nblk > 16) || nblk / p.S >= 12);
   p.xab = ((size_t)p.MTG * kBM * K * 2 + 255) & ~(size_t)255;
   p.tsb = ((size_t)p.MTG * kBM * 4 + 255) & ~(size_t)255;
   p.pb = p.R ? (size_t)(p.S - 1) * p.R * kTileElems * p.nt * 4 : 0;
