@@ -531,7 +531,11 @@ constexpr int gemm32s_wait(int fmt, int nt, bool deep, int c, int ahead) {
   }
   return n > 63 ? 63 : n;
 }
-template <int FMT, int WPE, int NTW, bool DEEP>
+// WIDE (rows of more than kMaxNarrowK values): the operand offsets of a 128-token tile, 256 bytes per value,
+// pass 31 bits, so the 64-bit base carries them. (On ordinary rows that form is slower: us, 77 / 512 tokens
+// of 18944 x 3584 32.2 / 81.5, with the base per super-block 32.5 / 81.8, per stage 32.3 / 82.0.)
+constexpr int kMaxNarrowK = 1 << 23;
+template <int FMT, int WPE, int NTW, bool DEEP, bool WIDE>
 __global__ __launch_bounds__(64 * kGemmWaves) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void quant_gemm32s_kernel(
     const uint8_t *__restrict__ W, const uint4 *__restrict__ xa,
     const float *__restrict__ tscale, float *__restrict__ Y, int N,
@@ -543,7 +547,6 @@ __global__ __launch_bounds__(64 * kGemmWaves) __attribute__((amdgpu_waves_per_eu
   constexpr int NT = NTW;                                       // 32-row MFMA tiles per wave
   constexpr int kBTn = 2 * NT * NW;                             // 16-row tiles per workgroup
   constexpr int kRT = 16 * kBTn;                                // rows per workgroup tile
-  constexpr int kDMA = 8 / NW;                                  // stage loads per wave
   // Four named arrays, not one indexed array: the compiler tracks LDS DMA per object, so a read
   // of one stage does not wait for the DMA into another.
   __shared__ u32x4 As0[kSU];
@@ -567,14 +570,15 @@ __global__ __launch_bounds__(64 * kGemmWaves) __attribute__((amdgpu_waves_per_eu
   const Magic K = magic_consts();
   const u32x4 *xg = reinterpret_cast<const u32x4 *>(xa) + (size_t)(4 * mg) * nq * 64;
   const int tile0 = kBTn * ng;
-  // Stage s = 8 b + 2 c + h: slices 16 (4 b + c) + h + 2 hi of token tile i at [(2 i + hi) * 64],
-  // one 1 KB wave load each; wave w loads units kDMA w .. kDMA w + kDMA - 1 (unit 2 i + hi).
-  const void *abase = xg;
+  // Stage s = chunk s of the range: K16 slice j of token tile i at [(4 i + j) * 64], one 1 KB load; wave w
+  // loads token tile w.
+  const uint8_t *abase = reinterpret_cast<const uint8_t *>(xg);
   const int off16 = 16 * lane;
-  auto load_stage = [&](int s, u32x4 *dst) {  // chunk s of the range: wave w loads token tile w's 4 K16 slices
-    const int so = (4 * kb0 + s) * 4096 + wave * nq * 1024;
+  auto load_stage = [&](int s, u32x4 *dst) {
+    const uint8_t *base = WIDE ? abase + (size_t)wave * nq * 1024 + ((size_t)4 * kb0 + s) * 4096 : abase;
+    const int so = WIDE ? 0 : (4 * kb0 + s) * 4096 + wave * nq * 1024;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) lds_load16(abase, dst + (4 * wave + j) * 64, off16, so + j * 1024);
+    for (int j = 0; j < 4; ++j) lds_load16(base, dst + (4 * wave + j) * 64, off16, so + j * 1024);
   };
   auto buf = [&](int k) -> u32x4 * { return k == 0 ? As0 : k == 1 ? As1 : k == 2 ? As2 : As3; };
 
@@ -985,13 +989,15 @@ int launch_gemm32(int fmt, const void *Wv, const float *X, float *Y, int N, int 
     return FHIP_OK;
   };
   const int grid2 = p.F + p.R * p.S;
+  const bool wide = K > kMaxNarrowK;
+  auto staged = [&](auto kern) {
+    kern<<<grid2, 64 * kGemmWaves, 0, stream()>>>(W, xa, ts, Y, N, M, nblk, ntiles, MTG, p.F, p.S, p.R, part);
+  };
   if (fmt == 1 && p.form != 1) {
     if (p.nt == 2)
-      quant_gemm32s_kernel<1, 2, 2, false><<<grid2, 64 * kGemmWaves, 0, stream()>>>(
-          W, xa, ts, Y, N, M, nblk, ntiles, MTG, p.F, p.S, p.R, part);
+      staged(wide ? quant_gemm32s_kernel<1, 2, 2, false, true> : quant_gemm32s_kernel<1, 2, 2, false, false>);
     else
-      quant_gemm32s_kernel<1, 3, 1, false><<<grid2, 64 * kGemmWaves, 0, stream()>>>(
-          W, xa, ts, Y, N, M, nblk, ntiles, MTG, p.F, p.S, p.R, part);
+      staged(wide ? quant_gemm32s_kernel<1, 3, 1, false, true> : quant_gemm32s_kernel<1, 3, 1, false, false>);
     FHIP_CHECK_LAUNCH("quant_gemm32s_kernel<1>");
     return reduce();
   }
@@ -1003,14 +1009,13 @@ int launch_gemm32(int fmt, const void *Wv, const float *X, float *Y, int N, int 
   }
   if (p.form != 1) {
     if (p.nt == 2)
-      quant_gemm32s_kernel<0, 2, 2, false><<<grid2, 64 * kGemmWaves, 0, stream()>>>(
-          W, xa, ts, Y, N, M, nblk, ntiles, MTG, p.F, p.S, p.R, part);
+      staged(wide ? quant_gemm32s_kernel<0, 2, 2, false, true> : quant_gemm32s_kernel<0, 2, 2, false, false>);
+    else if (wide)  // such a row's ranges are long whatever the grid
+      staged(quant_gemm32s_kernel<0, 2, 1, true, true>);
     else if (p.deep)
-      quant_gemm32s_kernel<0, 2, 1, true><<<grid2, 64 * kGemmWaves, 0, stream()>>>(
-          W, xa, ts, Y, N, M, nblk, ntiles, MTG, p.F, p.S, p.R, part);
+      staged(quant_gemm32s_kernel<0, 2, 1, true, false>);
     else
-      quant_gemm32s_kernel<0, 3, 1, false><<<grid2, 64 * kGemmWaves, 0, stream()>>>(
-          W, xa, ts, Y, N, M, nblk, ntiles, MTG, p.F, p.S, p.R, part);
+      staged(quant_gemm32s_kernel<0, 3, 1, false, false>);
     FHIP_CHECK_LAUNCH("quant_gemm32s_kernel<0>");
     return reduce();
   }
