@@ -91,14 +91,25 @@ struct W16<1> {
 template <int FMT>  // FMT 0: Q4_K, 1: Q6_K
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void quant_gemv16_kernel(
     const uint8_t *__restrict__ W, const float *__restrict__ X, float *__restrict__ Y,
-    float *__restrict__ part, int N, int K, int M, int nblk, int ntiles, int SK) {
+    float *__restrict__ part, int N, int K, int Mall, int nblk, int ntiles, int SK) {
   // Two stage buffers: the one being read and the one being built.
   __shared__ u32x4 As0[kUnitsSB * 64];
   __shared__ u32x4 As1[kUnitsSB * 64];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kap = lane >> 5, rho = lane & 31, r16 = rho & 15;
-  const int rb = blockIdx.x / SK, sp = blockIdx.x - rb * SK;
+  // More than 16 tokens: each (rows, range) has a workgroup for the first sixteen and one for the rest,
+  // eight apart, so on the same of the 8 XCDs (workgroups go to them in turn): the second's records come
+  // from its L2.
+  int id = blockIdx.x, t0 = 0;
+  if (Mall > 16) {
+    const int works = gridDim.x >> 1, g = id >> 4, n = min(8, works - 8 * g), j = id & 15;
+    t0 = j >= n ? 16 : 0;
+    id = 8 * g + (j >= n ? j - n : j);
+  }
+  const int M = min(16, Mall - t0);  // this workgroup's tokens, from t0
+  X += (size_t)t0 * K;
+  const int rb = id / SK, sp = id - rb * SK;
   const int kb0 = sp * nblk / SK, kb1 = (sp + 1) * nblk / SK;  // >= 1 super-block: SK <= nblk
   const int nb = kb1 - kb0;
   constexpr int NT = tiles16<FMT>();               // 32-row MFMA tiles per wave
@@ -473,9 +484,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       const int tok = 8 * (e >> 2) + 4 * kap + (e & 3);
       if (tok >= M) continue;
       if (SK == 1)
-        Y[(size_t)tok * N + row] = v[t][e];
+        Y[(size_t)(t0 + tok) * N + row] = v[t][e];
       else
-        part[((size_t)sp * M + tok) * N + row] = v[t][e];
+        part[((size_t)sp * Mall + t0 + tok) * N + row] = v[t][e];
     }
   }
 }
@@ -552,11 +563,6 @@ namespace {
 template <int FMT>
 int launch_gemv16(const void *Wv, const float *X, float *Y, int N, int K, int M) {
   if (M < 1 || M > 32) return fail(FHIP_EINVAL, "gemv16: M=%d outside 1..32", M);
-  // 17..32 tokens (only where a row is too long for q4k_mid.hip): sixteen, then the rest.
-  if (M > 16) {
-    if (int rc = launch_gemv16<FMT>(Wv, X, Y, N, K, 16)) return rc;
-    return launch_gemv16<FMT>(Wv, X + (size_t)16 * K, Y + (size_t)16 * N, N, K, M - 16);
-  }
   const int nblk = K / 256, ntiles = q4k_tiles(N);
   const int nrb = ceil_div(ntiles, 8 * tiles16<FMT>());
   const int SK = gemv16_splits(nblk);
@@ -567,7 +573,10 @@ int launch_gemv16(const void *Wv, const float *X, float *Y, int N, int K, int M)
     if (int rc = check_disjoint("gemv16", X, (size_t)M * K * 4, part, (size_t)SK * M * N * 4))
       return rc;
   }
-  quant_gemv16_kernel<FMT><<<nrb * SK, 256, 0, stream()>>>((const uint8_t *)Wv, X, Y, part, N, K,
+  // 17..32 tokens come only where a row is too long for q4k_mid.hip. Both halves in one launch (us at 17 /
+  // 32 tokens, two launches / one: Q4_K 3584 x 262400 354 / 384 -> 282 / 322, 40 x 262400 54 / 59 -> 38 /
+  // 38, Q6_K 40 x 262400 55 / 60 -> 37 / 38).
+  quant_gemv16_kernel<FMT><<<(M > 16 ? 2 : 1) * nrb * SK, 256, 0, stream()>>>((const uint8_t *)Wv, X, Y, part, N, K,
                                                             M, nblk, ntiles, SK);
   FHIP_CHECK_LAUNCH("quant_gemv16_kernel");
   if (SK > 1) return sum_ranges(part, Y, SK, M * N);

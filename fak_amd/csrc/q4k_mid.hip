@@ -378,6 +378,7 @@ __global__ __launch_bounds__(64 * NW) void quant_mid_kernel(const uint8_t *__res
 
 namespace {
 
+constexpr int kF16Row = 262144;  // rows longer than this take hi and lo operands up to 32 tokens
 constexpr int kMidRanges = 64;  // what sum_ranges reads at once
 // Operands (at most 36 MB, by mid_takes) and partial results together stay well inside the 64 MiB of the
 // no-allocation entry, whatever the shape.
@@ -403,17 +404,17 @@ constexpr MidPace kMidPace[2] = {{1.13f, 1.68f, 2.15f, 0.61f, 0.4f, 1.9f, 0.06f,
 MidPlan plan_mid(int fmt, int N, int K, int M, int TT, int NW) {
   MidPlan p{};
   const int nblk = K / 256, cus = cu_count() > 0 ? cu_count() : 256;
-  p.hl = M <= 16;
+  p.hl = M <= 16 || K > kF16Row;
   p.TT = TT;
   p.NW = NW;
-  p.MTG = p.hl ? 1 : ceil_div(M, 32 * TT);
-  p.tokens = p.hl ? 16 : 32 * TT * p.MTG;
+  p.MTG = p.hl ? ceil_div(M, 16) : ceil_div(M, 32 * TT);
+  p.tokens = p.hl ? 16 * p.MTG : 32 * TT * p.MTG;
   p.tasks = p.MTG * ceil_div(N, 32 * NW);
   const MidPace &m = kMidPace[fmt];
   const int fit = NW == 8 ? 1 : 2;  // workgroups per CU
-  p.xb = (size_t)(p.hl ? 1 : TT * p.MTG) * nblk * kSbUnits * 1024;
+  p.xb = (size_t)TT * p.MTG * nblk * kSbUnits * 1024;
   for (int sk = 1; sk <= nblk && sk <= kMidRanges; ++sk) {
-    if (sk > 1 && p.xb + (size_t)sk * M * N * 4 > kMidScratch) break;
+    if (sk > 1 && fmt == 0 && p.xb + (size_t)sk * M * N * 4 > kMidScratch) break;
     const long long wgs = (long long)p.tasks * sk;
     const float pace = fit == 1 ? m.wide : wgs <= cus ? m.one : m.two;
     const float rounds = wgs <= cus ? 1.f : (float)((wgs + fit * cus - 1) / (fit * cus));
@@ -450,7 +451,7 @@ namespace {
 // 18.4, 3584 x 25600 22.7 / 20.1.) 17..64: all. 65..128: matrices of up to w128 weights, whose prefill
 // GEMM runs too few tiles. Rows long enough to make the operands large keep the other kernels.
 bool mid_takes(int N, int K, int M, long long w128) {
-  if (K > 262144) return false;
+  if (K > kF16Row) return false;
   if (M <= 16) return K <= 24576 || N >= 3072;
   return M <= 64 || (M <= 128 && K <= 131072 && (long long)N * K <= w128);
 }
@@ -471,7 +472,13 @@ bool q4k_mid_takes(int N, int K, int M) {
 }
 
 // 65..128 tokens: 8192 x 2048 at 128 25.8 / 20.6, 1536 x 8192 20.8 / 17.9.
-bool q6k_mid_takes(int N, int K, int M) { return M >= 2 && mid_takes(N, K, M, 1 << 24); }
+// 17..32 tokens of more than a few rows of kF16Row to 2^20 values, whose two groups of 16 tokens read the
+// records through one L2 (us, q4k_gemv16.hip / this at 24 tokens: 3584 x 262400 524 / 377, 1000 x 262400
+// 156 / 132, 2000 x 524288 593 / 450; 40 x 262400 36.9 / 66.9, as 64 ranges leave it few workgroups).
+bool q6k_mid_takes(int N, int K, int M) {
+  if (K > kF16Row) return M > 16 && M <= 32 && N >= 512 && K <= 4 * kF16Row;
+  return M >= 2 && mid_takes(N, K, M, 1 << 24);
+}
 
 size_t mid_ws_bytes(int fmt, int N, int K, int M) {
   const MidPlan p = plan_mid(fmt, N, K, M);

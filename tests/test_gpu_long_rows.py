@@ -2,7 +2,10 @@
 but for a few super-blocks, so the reference (64 bits, the weights decoded on the host) needs those only.
 
 Tolerances, max|d|/RMS of a token's 16 outputs: f16 activations and f16-rounded weights (prefill GEMM),
-rounding errors independent: 3.7e-4 RMS of an output, and the largest of 80 under 4 times that: 2e-3."""
+rounding errors independent: 3.7e-4 RMS of an output, and the largest of 80 under 4 times that: 2e-3. Up
+to 32 tokens hi and lo operands (22 bits) and exact weights: 1e-5."""
+import time
+
 import numpy as np
 import pytest
 
@@ -53,3 +56,44 @@ def test_prefill_gemm(hip, fmt, in_, P):
     nb = in_ // 256
     check(fmt, 16, in_, P, [0, 3, 40, 99, P - 1] if P > 100 else [0, 3, 40, 99],
           [0, 1, nb // 2, nb - 2, nb - 1], 2e-3)
+
+
+@pytest.mark.parametrize("fmt,out,in_,P", [("q4k", 16, 262400, 17), ("q4k", 300, 262400, 32), ("q4k", 130, 1048832, 23),
+                                           ("q6k", 130, 262400, 18), ("q6k", 511, 262400, 31),
+                                           ("q6k", 530, 262400, 32), ("q6k", 600, 1048576, 17),
+                                           ("q6k", 513, 1048832, 20)])
+def test_17_to_32_tokens(hip, fmt, out, in_, P):
+    """Rows too long for the few-token kernel's f16 form: both sixteens of tokens, every range."""
+    print(f"[case] long rows {fmt} out={out} in={in_} P={P}", flush=True)
+    nb = in_ // 256
+    check(fmt, out, in_, P, sorted({0, 1, 15, 16, P - 1}), [0, 1, 2, 5, nb // 2, nb // 2 + 1, nb - 1], 1e-5)
+
+
+def seconds(prefix, w, out, in_, P):
+    with Dev(P * in_ * 4) as dx, Dev(P * out * 4) as dy:
+        fakhip.call("fhip_memset_async", dx.ptr, 0, dx.nbytes)
+        best = 1e9
+        for _ in range(5):
+            fakhip.call("fhip_sync")
+            t = time.perf_counter()
+            for _ in range(4):
+                fakhip.call(prefix + "_matmul_f32", w, dx.ptr, dy.ptr, out, in_, P)
+            fakhip.call("fhip_sync")
+            best = min(best, time.perf_counter() - t)
+    return best
+
+
+@pytest.mark.parametrize("fmt,out,in_,few,many,bound", [("q4k", 40, 262400, 16, 32, 1.65),
+                                                        ("q6k", 40, 262400, 16, 32, 1.65)])
+def test_many_tokens_read_the_rows_together(hip, fmt, out, in_, few, many, bound):
+    """Tokens one after the other, or in groups one after the other, would take `many` / `few` times as long."""
+    print(f"[case] long rows, time of {many} tokens against {few}, {fmt} in={in_}", flush=True)
+    prefix, size, block = ENTRY[fmt][:3]
+    lib = fakhip.load()
+    raw = np.zeros(out * (in_ // block) * size, np.uint8)
+    w = fakhip.alloc_call(prefix + "_upload", raw.ctypes.data, out, in_)
+    try:
+        seconds(prefix, w, out, in_, many)  # workspaces, clocks
+        assert seconds(prefix, w, out, in_, many) < bound * seconds(prefix, w, out, in_, few)
+    finally:
+        lib.fhip_free(w)
