@@ -10,17 +10,18 @@ import numpy as np
 import pytest
 
 from fak_amd import fakhip, synth
-from tests import test_gpu_q4k_mid as q4k, test_gpu_q6k_mid as q6k
+from tests import test_gpu_q4k_mid as q4k, test_gpu_q6k_mid as q6k, test_gpu_q8_0_gemm as q8_0
 from tests.gpu_util import Dev, rel_err_rows
 
 pytestmark = pytest.mark.gpu
 
 ENTRY = {"q4k": ("fhip_q4k", 144, 256, q4k.exact, lambda o, i: synth.q4k_weights(o, i, 5)),
+         "q8_0": ("fhip_q8_0", 34, 32, q8_0.exact, lambda o, i: synth.q8_0_weights(o, i, 5)),
          "q6k": ("fhip_q6k", 210, 256, q6k.exact, lambda o, i: q6k.weights(o, i, 5))}
 
 
 def check(fmt, out, in_, P, tokens, blocks, tol):
-    """Tokens `tokens` are N(0, 1) in the blocks (of the format's 256 values) `blocks`, all else is zero."""
+    """Tokens `tokens` are N(0, 1) in the blocks (of the format: 256 or 32 values) `blocks`, all else is zero."""
     prefix, size, block, exact, weights = ENTRY[fmt]
     lib = fakhip.load()
     nb, n = in_ // block, len(blocks)
@@ -69,6 +70,16 @@ def test_17_to_32_tokens(hip, fmt, out, in_, P):
     check(fmt, out, in_, P, sorted({0, 1, 15, 16, P - 1}), [0, 1, 2, 5, nb // 2, nb // 2 + 1, nb - 1], 1e-5)
 
 
+@pytest.mark.parametrize("out,in_,P", [(33, 1 << 21, 40), (33, (1 << 21) + 32, 2), (17, (1 << 21) + 64, 16),
+                                       (50, (1 << 21) + 32, 35)])
+def test_q8_0(hip, out, in_, P):
+    """The longest row of the GEMM, and rows past it: the GEMV in slices of sixteen tokens. Its per-row
+    rounding (products of 1152 + code less 1152 times the sum) is a few 2^-20: 2e-5."""
+    print(f"[case] long rows q8_0 out={out} in={in_} P={P}", flush=True)
+    nb = in_ // 32
+    check("q8_0", out, in_, P, sorted({0, 1, P - 1}), [0, 1, 7, 8, nb // 2, nb // 2 + 1, nb - 2, nb - 1], 2e-5)
+
+
 def seconds(prefix, w, out, in_, P):
     with Dev(P * in_ * 4) as dx, Dev(P * out * 4) as dy:
         fakhip.call("fhip_memset_async", dx.ptr, 0, dx.nbytes)
@@ -84,7 +95,8 @@ def seconds(prefix, w, out, in_, P):
 
 
 @pytest.mark.parametrize("fmt,out,in_,few,many,bound", [("q4k", 40, 262400, 16, 32, 1.65),
-                                                        ("q6k", 40, 262400, 16, 32, 1.65)])
+                                                        ("q6k", 40, 262400, 16, 32, 1.65),
+                                                        ("q8_0", 16, 2097184, 1, 16, 6)])
 def test_many_tokens_read_the_rows_together(hip, fmt, out, in_, few, many, bound):
     """Tokens one after the other, or in groups one after the other, would take `many` / `few` times as long."""
     print(f"[case] long rows, time of {many} tokens against {few}, {fmt} in={in_}", flush=True)

@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from fak_amd import synth
-from tests.gpu_util import q8_0_matmul, rel_err_rows, scaled_activations
+from tests.gpu_util import knobs, q8_0_matmul, rel_err_rows, scaled_activations
 
 pytestmark = pytest.mark.gpu
 
@@ -46,3 +46,15 @@ def test_scales_and_special_values(hip, pattern):
     keep = [t for t in range(P) if t not in (7, 20)]
     # a row of one huge value is held to its RMS: 22 bits below it
     assert rel_err_rows(Y[keep], ref[keep]) <= 1e-5
+
+
+@pytest.mark.parametrize("out,in_,P", [(200, 2048, 8), (33, 1056, 16), (3584, 3584, 3)])
+def test_gemv_global_operands_forced(hip, monkeypatch, out, in_, P):
+    """FAK_HIP_GEMV_GLOBALX=1: the GEMV with its operands in global memory, up to 16 tokens. Products of
+    1152 + code less 1152 times the sum: a few 2^-20."""
+    print(f"[case] q8_0 gemv global operands out={out} in={in_} P={P}", flush=True)
+    raw = synth.q8_0_weights(out, in_, seed=out + in_)
+    X = synth.activations(P, in_, P)
+    with knobs(monkeypatch, FAK_HIP_GEMV_GLOBALX=1):
+        Y = q8_0_matmul(raw, out, in_, X, P)
+    assert rel_err_rows(Y, exact(raw, out, in_, X)) <= 2e-5
