@@ -449,8 +449,11 @@ int fhip_q8_0_matmul_f32(const void *dPacked, const float *dX, float *dY, int ou
     return FHIP_OK;
   }
   if (q8_takes_gemv(out, in, P)) return q8_0_gemv(dPacked, dX, dY, out, in, P);
-  for (int t0 = 0; t0 < P; t0 += kQ8GemmTokens) {
-    const int m = P - t0 < kQ8GemmTokens ? P - t0 : kQ8GemmTokens;
+  // Slices whose operands (4 bytes per value) stay within 256 MiB: 1024 tokens up to 65536 values, 32 of the
+  // longest rows, where 1024 would take 8.6 GB of scratch.
+  const int slice = min(kQ8GemmTokens, ((64 << 20) / in) & ~31);
+  for (int t0 = 0; t0 < P; t0 += slice) {
+    const int m = P - t0 < slice ? P - t0 : slice;
     if (int rc = q8_0_gemm(dPacked, dX + (size_t)t0 * in, dY + (size_t)t0 * out, out, in, m))
       return rc;
   }

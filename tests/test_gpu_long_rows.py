@@ -4,6 +4,7 @@ but for a few super-blocks, so the reference (64 bits, the weights decoded on th
 Tolerances, max|d|/RMS of a token's 16 outputs: f16 activations and f16-rounded weights (prefill GEMM),
 rounding errors independent: 3.7e-4 RMS of an output, and the largest of 80 under 4 times that: 2e-3. Up
 to 32 tokens hi and lo operands (22 bits) and exact weights: 1e-5."""
+import ctypes as C
 import time
 
 import numpy as np
@@ -78,6 +79,32 @@ def test_q8_0(hip, out, in_, P):
     print(f"[case] long rows q8_0 out={out} in={in_} P={P}", flush=True)
     nb = in_ // 32
     check("q8_0", out, in_, P, sorted({0, 1, P - 1}), [0, 1, 7, 8, nb // 2, nb // 2 + 1, nb - 2, nb - 1], 2e-5)
+
+
+@pytest.mark.parametrize("in_,P", [(1 << 20, 130), ((1 << 19) + 32, 300), (65536, 1000)])
+def test_q8_0_scratch(hip, in_, P):
+    """A wide call of a long row keeps its scratch within 256 MiB (and the workspace's quarter over it)."""
+    print(f"[case] long rows q8_0 scratch in={in_} P={P}", flush=True)
+    lib, free, total = fakhip.load(), C.c_size_t(), C.c_size_t()
+    raw = np.zeros(40 * (in_ // 32) * 34, np.uint8)
+    w = fakhip.alloc_call("fhip_q8_0_upload", raw.ctypes.data, 40, in_)
+    st = C.c_void_p()  # a stream of its own: its workspace starts empty
+    fakhip.call("fhip_stream_create", C.byref(st))
+    fakhip.call("fhip_set_stream", st)
+    try:
+        with Dev(P * in_ * 4) as dx, Dev(P * 40 * 4) as dy:
+            fakhip.call("fhip_mem_info", C.byref(free), C.byref(total))
+            before = free.value
+            fakhip.call("fhip_q8_0_matmul_f32", w, dx.ptr, dy.ptr, 40, in_, P)
+            fakhip.call("fhip_sync")
+            fakhip.call("fhip_mem_info", C.byref(free), C.byref(total))
+    finally:
+        fakhip.call("fhip_set_stream", None)
+        fakhip.call("fhip_stream_destroy", st)
+        lib.fhip_free(w)
+        lib.fhip_trim_pool(0)
+    # scales and the partial sums of the K ranges, at most 32 MiB, come on top
+    assert before - free.value <= 1.25 * (288 << 20)
 
 
 def seconds(prefix, w, out, in_, P):
