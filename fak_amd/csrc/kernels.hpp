@@ -238,6 +238,19 @@ __device__ __forceinline__ uint32_t absmax4_bits(float x0, float x1, float x2, f
              max(__float_as_uint(x2) & m, __float_as_uint(x3) & m));
 }
 
+// Lane exchanges on the VALU (DPP), where __shfl_xor goes through LDS: with lane ^ 1 or lane ^ 2, and the
+// mirror of a group of 8 or 16 lanes (a reduction whose halves of the group are uniform needs no more).
+template <int O>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
+  static_assert(O == 1 || O == 2, "within four lanes");
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, O == 1 ? 0xB1 : 0x4E, 0xf, 0xf, true);  // quad_perm
+}
+template <int G>
+__device__ __forceinline__ uint32_t group_mirror(uint32_t v) {
+  static_assert(G == 8 || G == 16, "row_half_mirror, row_mirror");
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, G == 8 ? 0x141 : 0x140, 0xf, 0xf, true);
+}
+
 // Workgroup shape of the small-M GEMV kernels (TW tiles x KW waves; see q4k_gemv.hip).
 void gemv_shape(int ntiles, int nblk, int max_waves, size_t lds_fixed, size_t lds_per_wave,
                 int &TW, int &KW);

@@ -48,6 +48,27 @@ def test_scales_and_special_values(hip, pattern):
     assert rel_err_rows(Y[keep], ref[keep]) <= 1e-5
 
 
+@pytest.mark.parametrize("out,in_,P", [(200, 2048, 40), (129, 96, 33), (2100, 4096, 150), (40, 18944, 96),
+                                       (513, 3616, 200)])
+def test_small_blocks_beside_large_ones(hip, out, in_, P):
+    """Blocks far below their range's largest magnitude are all an output sees where the larger blocks
+    meet zero weights: they keep their 22 bits, at every ratio, in the tokens that have them and in
+    ordinary tokens of the same tile."""
+    print(f"[case] q8_0 gemm small beside large out={out} in={in_} P={P}", flush=True)
+    raw = synth.q8_0_weights(out, in_, seed=out + in_).reshape(out, in_ // 32, 34)
+    big = np.arange(in_ // 32) % 3 == 1
+    raw[:, big, 2:] = 0
+    X = synth.activations(P, in_, P).reshape(P, in_ // 32, 32)
+    ratios = [1.0, 2.0 ** 12, 2.0 ** 16, 1e6, 1e24, 1e30]
+    for t in range(P):
+        X[t, big] *= np.float32(ratios[t % 6])
+        X[t] *= np.float32([1.0, 1e-3, 1.0, 1e-20, 1e-20, 1e-34][t % 6])
+    X[3, 0, :] = 0.0
+    X = X.reshape(P, in_)
+    raw = raw.reshape(-1)
+    assert rel_err_rows(q8_0_matmul(raw, out, in_, X, P), exact(raw, out, in_, X)) <= 1e-5
+
+
 @pytest.mark.parametrize("out,in_,P", [(200, 2048, 8), (33, 1056, 16), (3584, 3584, 3)])
 def test_gemv_global_operands_forced(hip, monkeypatch, out, in_, P):
     """FAK_HIP_GEMV_GLOBALX=1: the GEMV with its operands in global memory, up to 16 tokens. Products of
