@@ -6,7 +6,9 @@
 // term is one more MFMA over the sub-block sums, and activations are scaled by a power of two per
 // (token, K range) that puts the range's largest magnitude in [2^13, 2^14). Up to 16 tokens the 32
 // operand rows are the f16 of each value and the f16 of its remainder (~22 bits); above, 32 tokens in
-// f16.
+// f16. A range with a super-block whose largest magnitude lies 2^13 and more below the range's has a scale
+// per super-block instead (up to 32 tokens), applied to the super-block's sum: the range's would leave such
+// values too few bits, or none, and they are all there is where the weights of the larger ones are zero.
 //
 // The data path is another: the operands are made once per call (mid_xprep_kernel), not by every
 // workgroup, and every workgroup streams them and its weight records to LDS by direct loads two
@@ -45,52 +47,78 @@ constexpr int kSbUnits = 17;
 template <bool HL, int UPT>
 __global__ __launch_bounds__(256) void mid_xprep_kernel(const float *__restrict__ X, int M, int K, int nblk,
                                                         int SK, u32x4 *__restrict__ xa,
-                                                        float *__restrict__ tscale) {
-  __shared__ uint32_t wmax[4];
+                                                        float *__restrict__ tscale,
+                                                        float *__restrict__ bscale) {
+  __shared__ uint32_t wmax[4], wmin[4];
   const int tokens = gridDim.x, t = blockIdx.x, sp = blockIdx.y, tid = threadIdx.x;
   const int u0 = 32 * (sp * nblk / SK), u1 = 32 * ((sp + 1) * nblk / SK);
   const bool valid = t < M;
   const float4 *row = reinterpret_cast<const float4 *>(X + (size_t)(valid ? t : 0) * K);
-  uint32_t m = 0;
+  uint32_t m = 0, mn = ~0u;  // largest magnitude, and smallest of a super-block's that are not zero
   float4 reg[UPT > 0 ? UPT : 1][2];
-  auto see = [&](const float4 v) { m = max(m, absmax4_bits(v.x, v.y, v.z, v.w)); };
+  // Largest magnitude of a super-block: its 32 units are half a wave's.
+  auto block_max = [](const float4 a, const float4 c) {
+    uint32_t w = max(absmax4_bits(a.x, a.y, a.z, a.w), absmax4_bits(c.x, c.y, c.z, c.w));
+    w = max(w, lane_xor<1>(w));
+    w = max(w, lane_xor<2>(w));
+    w = max(w, group_mirror<8>(w));
+    w = max(w, group_mirror<16>(w));
+    return max(w, (uint32_t)__shfl_xor((int)w, 16));
+  };
+  auto see = [&](const uint32_t w) {
+    m = max(m, w);
+    mn = min(mn, w - 1);  // zero last
+  };
+  auto real = [&](int u) { return u < u1 ? u : u1 - 32 + (u & 31); };  // repeats do not change either
   if (UPT > 0) {
 #pragma unroll
     for (int j = 0; j < UPT; ++j) {
-      const int u = min(u0 + tid + 256 * j, u1 - 1);
+      const int u = real(u0 + tid + 256 * j);
       reg[j][0] = row[2 * u];
       reg[j][1] = row[2 * u + 1];
     }
 #pragma unroll
-    for (int j = 0; j < UPT; ++j) {
-      see(reg[j][0]);
-      see(reg[j][1]);
-    }
+    for (int j = 0; j < UPT; ++j) see(block_max(reg[j][0], reg[j][1]));
   } else {
-    for (int u = u0 + tid; u < u1; u += 256) {
-      see(row[2 * u]);
-      see(row[2 * u + 1]);
-    }
+    for (int u = u0 + tid; u < u1; u += 256) see(block_max(row[2 * u], row[2 * u + 1]));
   }
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o));
-  if ((tid & 63) == 0) wmax[tid >> 6] = m;
+  m = max(m, (uint32_t)__shfl_xor((int)m, 32));
+  mn = min(mn, (uint32_t)__shfl_xor((int)mn, 32));
+  if ((tid & 63) == 0) {
+    wmax[tid >> 6] = m;
+    wmin[tid >> 6] = mn;
+  }
   __syncthreads();
   m = valid ? max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3])) : 0u;
+  mn = min(min(wmin[0], wmin[1]), min(wmin[2], wmin[3])) + 1;
   const bool finite = m < 0x7F800000u;
-  int e = 0;
-  (void)frexpf(__uint_as_float(m), &e);
-  const int k = finite ? e - 14 : 0;
-  if (tid == 0) tscale[(size_t)sp * tokens + t] = !finite ? __builtin_nanf("") : m ? ldexpf(1.f, k) : 1.f;
+  // The exponent that puts w in [2^13, 2^14), at least -126: 2^k stays normal, and the bits of magnitudes
+  // below 2^-112 all fit in the operands.
+  auto exponent = [](uint32_t w) {
+    int e = 0;
+    (void)frexpf(__uint_as_float(w), &e);
+    return max(e - 14, -126);
+  };
+  const int k = finite && m ? exponent(m) : 0;
+  const bool fine = bscale && finite && m && (m >> 23) > (mn >> 23) + 13;
+  // -1: the scales are the super-blocks'
+  if (tid == 0) tscale[(size_t)sp * tokens + t] = !finite ? __builtin_nanf("") : fine ? -1.f : ldexpf(1.f, k);
   constexpr int TPT = HL ? 16 : 32;  // tokens per operand tile
   const int tile = t / TPT, r = t % TPT;
   auto put = [&](int u, const float4 a, const float4 c) {
     const float v[8] = {a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
     const bool live = valid && finite;
+    const int b = u >> 5, q = u & 31;
+    int kb = k;
+    if (fine) {  // uniform over the workgroup
+      const uint32_t w = block_max(a, c);
+      kb = w ? exponent(w) : 0;
+      if (q == 0) bscale[((size_t)tile * nblk + b) * TPT + r] = ldexpf(1.f, kb);
+    }
     float s[8], sum = 0.f;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      s[j] = live ? ldexpf(v[j], -k) : 0.f;
+      s[j] = live ? ldexpf(v[j], -kb) : 0.f;
       sum += s[j];
     }
     f16x8 hi, lo;
@@ -99,7 +127,6 @@ __global__ __launch_bounds__(256) void mid_xprep_kernel(const float *__restrict_
       hi[j] = (_Float16)s[perm8(j)];
       lo[j] = (_Float16)(s[perm8(j)] - (float)hi[j]);
     }
-    const int b = u >> 5, q = u & 31;
     u32x4 *d = xa + ((size_t)tile * nblk + b) * (kSbUnits * 64);
     d[(q >> 1) * 64 + 32 * (q & 1) + r] = __builtin_bit_cast(u32x4, hi);
     if (HL) d[(q >> 1) * 64 + 32 * (q & 1) + 16 + r] = __builtin_bit_cast(u32x4, lo);
@@ -141,10 +168,13 @@ constexpr int wait_vm_mid(int n) { return 0x0070 | (n & 15) | ((n >> 4) << 14); 
 // Workgroup = NW waves x 32 rows x TT operand tiles over one K range. A stage is half a super-block:
 // 8 operand units per tile, shared by the waves, and each wave's two record parts; three buffers, each
 // stage loaded two ahead. The super-block's headers and sum units come with its first half.
+// The wave count is what the LDS allows; stated, it keeps the super-block results that the VALU scales in
+// VGPRs (the compiler had taken AGPRs for one operand tile).
 template <int FMT, int TT, bool HL, int NW>  // FMT 0: Q4_K, 1: Q6_K
-__global__ __launch_bounds__(64 * NW) void quant_mid_kernel(const uint8_t *__restrict__ W,
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void quant_mid_kernel(const uint8_t *__restrict__ W,
                                                             const u32x4 *__restrict__ xa,
                                                             const float *__restrict__ tscale,
+                                                            const float *__restrict__ bscale,
                                                             float *__restrict__ Y, float *__restrict__ part,
                                                             int N, int M, int nblk, int ntiles, int MTG,
                                                             int tokens, int SK) {
@@ -200,6 +230,8 @@ __global__ __launch_bounds__(64 * NW) void quant_mid_kernel(const uint8_t *__res
   for (int i = 0; i < TT; ++i)
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[i][e] = 0.f;
+  constexpr int TPT = HL ? 16 : 32, NV = HL ? 8 : 16;  // tokens per operand tile, of them a lane's
+  const float tsl = TT == 1 ? tscale[(size_t)sp * tokens + TPT * mg + (lane & (TPT - 1))] : 0.f;
   load(0, 0, S0, H0);
   load(0, 1, S1, nullptr);
   FHIP_LDS_BARRIER_MID(wait_vm_mid(0));
@@ -220,138 +252,169 @@ __global__ __launch_bounds__(64 * NW) void quant_mid_kernel(const uint8_t *__res
   const h2 k1152 = {(_Float16)1152.f, (_Float16)1152.f}, k4th = {(_Float16)0.25f, (_Float16)0.25f};
   const h2 k64th = k16th * k4th, kTb = {(_Float16)0.0625f, (_Float16)0.015625f};  // b under 2^6, 2^8
   const h2 kOb = {(_Float16)-72.f, (_Float16)-24.f};  // -(1024 + 2 2^6) / 16, -(1024 + 2 2^8) / 64
-  for (int bb = 0; bb < nb; bb += 3) {
+  auto range = [&](auto fine) {  // fine: with super-block scales
+    for (int bb = 0; bb < nb; bb += 3) {
 #pragma unroll
-    for (int u = 0; u < 6; ++u) {
-      const int b = bb + u / 2, hh = u & 1;
-      load(b + 1, hh, sbuf((u + 2) % 3), hbuf((u / 2 + 1) % 3));
-      if (b < nb) {
-        const u32x4 *Sb = sbuf(u % 3), *Hb = hbuf(u / 2);
-        if constexpr (FMT == 0) {
-          // the super-block's scales (read again at each half: cheaper than held registers)
-          const u32x4 hd = Hb[hl];
-          const uint32_t sc4 = hh == 0 ? hd[1] & 0x3F3F3F3Fu : (hd[3] & 0x0F0F0F0Fu) | ((hd[1] >> 2) & 0x30303030u);
-          const h2 ep = as_h2((sc4 & kB02) | kMagic) - k1024;         // sub-blocks 4 hh, 4 hh + 2
-          const h2 op = as_h2(((sc4 >> 8) & kB02) | kMagic) - k1024;  // 4 hh + 1, 4 hh + 3
-          const u32x4 nb0 = Sb[wl], nb1 = Sb[wl + 32];
-  #pragma unroll
-          for (int c = 0; c < 2; ++c) {
-            const _Float16 sa = c ? ep.y : ep.x, sb = c ? op.y : op.x;
-            const h2 SL = {sa, sa}, SH = h2{sb, sb} * k16th;
-            const h2 NL = SL * kN1024, NH = SH * kN1024;
-  #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-              const u32x4 q = h ? nb1 : nb0;
-              const uint32_t x0 = c ? q[2] : q[0], x1 = c ? q[3] : q[1];
-              const uint32_t y0 = x0 >> 8, y1 = x1 >> 8;
-              u32x4 lw, hw;
-              lw[0] = as_u(__builtin_elementwise_fma(as_h2((x0 & kLo) | kMagic), SL, NL));
-              lw[1] = as_u(__builtin_elementwise_fma(as_h2((y0 & kLo) | kMagic), SL, NL));
-              lw[2] = as_u(__builtin_elementwise_fma(as_h2((x1 & kLo) | kMagic), SL, NL));
-              lw[3] = as_u(__builtin_elementwise_fma(as_h2((y1 & kLo) | kMagic), SL, NL));
-              hw[0] = as_u(__builtin_elementwise_fma(as_h2((x0 & kHi) | kMagic), SH, NH));
-              hw[1] = as_u(__builtin_elementwise_fma(as_h2((y0 & kHi) | kMagic), SH, NH));
-              hw[2] = as_u(__builtin_elementwise_fma(as_h2((x1 & kHi) | kMagic), SH, NH));
-              hw[3] = as_u(__builtin_elementwise_fma(as_h2((y1 & kHi) | kMagic), SH, NH));
-  #pragma unroll
-              for (int hi = 0; hi < 2; ++hi)
-  #pragma unroll
-                for (int i = 0; i < TT; ++i) {
-                  const f16x8 a = __builtin_bit_cast(f16x8, Sb[(i * 8 + 4 * c + 2 * hi + h) * 64 + al]);
-                  f32x16 z = tmp[i][hi];
-                  if (hh == 0 && c == 0 && h == 0)
-  #pragma unroll
-                    for (int e = 0; e < 16; ++e) z[e] = 0.f;
-                  tmp[i][hi] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, __builtin_bit_cast(f16x8, hi ? hw : lw), z, 0, 0, 0);
-                }
-            }
-          }
-          if (hh == 1) {
-            const float d = (float)__builtin_bit_cast(_Float16, (uint16_t)(hd[0] & 0xffffu));
-            const float dm = (float)__builtin_bit_cast(_Float16, (uint16_t)(hd[0] >> 16));
-            const uint32_t mnl = hd[2] & 0x3F3F3F3Fu;
-            const uint32_t mnh = ((hd[3] >> 4) & 0x0F0F0F0Fu) | ((hd[2] >> 2) & 0x30303030u);
-            u32x4 mw;
-            mw[0] = as_u((as_h2((mnl & kB02) | kMagic) - k1024) * k32);
-            mw[1] = as_u((as_h2(((mnl >> 8) & kB02) | kMagic) - k1024) * k32);
-            mw[2] = as_u((as_h2((mnh & kB02) | kMagic) - k1024) * k32);
-            mw[3] = as_u((as_h2(((mnh >> 8) & kB02) | kMagic) - k1024) * k32);
-  #pragma unroll
-            for (int i = 0; i < TT; ++i) {
-              f32x16 mt;
-  #pragma unroll
-              for (int e = 0; e < 16; ++e) mt[e] = 0.f;
-              mt = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, Hb[(NW + i) * 64 + al]),
-                                                          __builtin_bit_cast(f16x8, mw), mt, 0, 0, 0);
-  #pragma unroll
-              for (int e = 0; e < 16; ++e)
-                acc[i][e] = fmaf(d, tmp[i][0][e] + tmp[i][1][e], fmaf(-dm, mt[e], acc[i][e]));
-            }
-          }
-        } else {
-          // Q6_K: group g = K16 slice g. With q = n + 16 b (nibble n, qh field b), sc_g (q - 32) / 4 is the
-          // sum of two operands that f16 holds exactly, sc_g n / 4 (up to 480) and 4 sc_g (b - 2) (up to
-          // 1024), each one fma of the field under the exponent of 1024 (n 2^(4 c), b 2^(6 + 2 hi)). Both
-          // feed one chain, whose running sum is that of the whole weights: with a chain each the error
-          // against 64 bits is 4% larger.
-          const uint2 *Q = reinterpret_cast<const uint2 *>(Sb);
-          const u32x4 hd = Hb[hl];
+      for (int u = 0; u < 6; ++u) {
+        const int b = bb + u / 2, hh = u & 1;
+        load(b + 1, hh, sbuf((u + 2) % 3), hbuf((u / 2 + 1) % 3));
+        if (b < nb) {
+          const u32x4 *Sb = sbuf(u % 3), *Hb = hbuf(u / 2);
+          float bs[NV];  // this super-block's scales, 1 for tokens whose range has one scale
+          if constexpr (decltype(fine)::value) {
+            if (hh == 1) {
 #pragma unroll
-          for (int c = 0; c < 2; ++c) {
-            const uint32_t sw = hd[2 * hh + c] ^ k80;
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-              const h2 P = as_h2(((h ? sw >> 8 : sw) & kB02) | kMagic) - k1152;  // scales of hi = 0, 1
-              const h2 SP = P * (c ? k64th : k4th), NP = SP * kN1024, TP = P * kTb, OP = P * kOb;
-              const uint2 qa = Q[ql + 32 * h], qb = Q[ql + 64 + 32 * h], qh = Q[qq + 32 * h];
-#pragma unroll
-              for (int hi = 0; hi < 2; ++hi) {
-                const _Float16 s = hi ? SP.y : SP.x, n = hi ? NP.y : NP.x, t = hi ? TP.y : TP.x, o = hi ? OP.y : OP.x;
-                const h2 S = {s, s}, N0 = {n, n}, T = {t, t}, O = {o, o};
-                const uint32_t mn = c ? kHi : kLo, mb = hi ? kB8 : kB6;
-                u32x4 vn, vb;
-#pragma unroll
-                for (int m = 0; m < 2; ++m) {
-                  const uint32_t x = hi ? (m ? qb.y : qb.x) : (m ? qa.y : qa.x), b4 = m ? qh.y : qh.x;
-                  const uint32_t be = b4 << (c ? 2 : 6), bo = b4 >> (c ? 6 : 2);
-                  vn[2 * m] = as_u(__builtin_elementwise_fma(as_h2((x & mn) | kMagic), S, N0));
-                  vn[2 * m + 1] = as_u(__builtin_elementwise_fma(as_h2(((x >> 8) & mn) | kMagic), S, N0));
-                  vb[2 * m] = as_u(__builtin_elementwise_fma(as_h2((be & mb) | kMagic), T, O));
-                  vb[2 * m + 1] = as_u(__builtin_elementwise_fma(as_h2((bo & mb) | kMagic), T, O));
-                }
-#pragma unroll
-                for (int i = 0; i < TT; ++i) {
-                  const f16x8 a = __builtin_bit_cast(f16x8, Sb[(i * 8 + 4 * c + 2 * hi + h) * 64 + al]);
-                  f32x16 z = tmp[i][hi];
-                  if (hh == 0 && c == 0 && h == 0)
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) z[e] = 0.f;
-                  z = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, __builtin_bit_cast(f16x8, vn), z, 0, 0, 0);
-                  tmp[i][hi] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, __builtin_bit_cast(f16x8, vb), z, 0, 0, 0);
-                }
+              for (int a = 0; a < NV / 4; ++a) {
+                const int r = 8 * a + 4 * kap;
+                const float4 s4 = *reinterpret_cast<const float4 *>(
+                    bscale + ((size_t)mg * nblk + b0 + b) * TPT + r);
+                const float4 t4 = *reinterpret_cast<const float4 *>(tscale + (size_t)sp * tokens + TPT * mg + r);
+                bs[4 * a] = t4.x < 0.f ? s4.x : 1.f;
+                bs[4 * a + 1] = t4.y < 0.f ? s4.y : 1.f;
+                bs[4 * a + 2] = t4.z < 0.f ? s4.z : 1.f;
+                bs[4 * a + 3] = t4.w < 0.f ? s4.w : 1.f;
               }
             }
           }
-          if (hh == 1) {
-            const float d = 4.f * (float)reinterpret_cast<const _Float16 *>(Hb)[dl];
+          if constexpr (FMT == 0) {
+            // the super-block's scales (read again at each half: cheaper than held registers)
+            const u32x4 hd = Hb[hl];
+            const uint32_t sc4 = hh == 0 ? hd[1] & 0x3F3F3F3Fu : (hd[3] & 0x0F0F0F0Fu) | ((hd[1] >> 2) & 0x30303030u);
+            const h2 ep = as_h2((sc4 & kB02) | kMagic) - k1024;         // sub-blocks 4 hh, 4 hh + 2
+            const h2 op = as_h2(((sc4 >> 8) & kB02) | kMagic) - k1024;  // 4 hh + 1, 4 hh + 3
+            const u32x4 nb0 = Sb[wl], nb1 = Sb[wl + 32];
+    #pragma unroll
+            for (int c = 0; c < 2; ++c) {
+              const _Float16 sa = c ? ep.y : ep.x, sb = c ? op.y : op.x;
+              const h2 SL = {sa, sa}, SH = h2{sb, sb} * k16th;
+              const h2 NL = SL * kN1024, NH = SH * kN1024;
+    #pragma unroll
+              for (int h = 0; h < 2; ++h) {
+                const u32x4 q = h ? nb1 : nb0;
+                const uint32_t x0 = c ? q[2] : q[0], x1 = c ? q[3] : q[1];
+                const uint32_t y0 = x0 >> 8, y1 = x1 >> 8;
+                u32x4 lw, hw;
+                lw[0] = as_u(__builtin_elementwise_fma(as_h2((x0 & kLo) | kMagic), SL, NL));
+                lw[1] = as_u(__builtin_elementwise_fma(as_h2((y0 & kLo) | kMagic), SL, NL));
+                lw[2] = as_u(__builtin_elementwise_fma(as_h2((x1 & kLo) | kMagic), SL, NL));
+                lw[3] = as_u(__builtin_elementwise_fma(as_h2((y1 & kLo) | kMagic), SL, NL));
+                hw[0] = as_u(__builtin_elementwise_fma(as_h2((x0 & kHi) | kMagic), SH, NH));
+                hw[1] = as_u(__builtin_elementwise_fma(as_h2((y0 & kHi) | kMagic), SH, NH));
+                hw[2] = as_u(__builtin_elementwise_fma(as_h2((x1 & kHi) | kMagic), SH, NH));
+                hw[3] = as_u(__builtin_elementwise_fma(as_h2((y1 & kHi) | kMagic), SH, NH));
+    #pragma unroll
+                for (int hi = 0; hi < 2; ++hi)
+    #pragma unroll
+                  for (int i = 0; i < TT; ++i) {
+                    const f16x8 a = __builtin_bit_cast(f16x8, Sb[(i * 8 + 4 * c + 2 * hi + h) * 64 + al]);
+                    f32x16 z = tmp[i][hi];
+                    if (hh == 0 && c == 0 && h == 0)
+    #pragma unroll
+                      for (int e = 0; e < 16; ++e) z[e] = 0.f;
+                    tmp[i][hi] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, __builtin_bit_cast(f16x8, hi ? hw : lw), z, 0, 0, 0);
+                  }
+              }
+            }
+            if (hh == 1) {
+              const float d = (float)__builtin_bit_cast(_Float16, (uint16_t)(hd[0] & 0xffffu));
+              const float dm = (float)__builtin_bit_cast(_Float16, (uint16_t)(hd[0] >> 16));
+              const uint32_t mnl = hd[2] & 0x3F3F3F3Fu;
+              const uint32_t mnh = ((hd[3] >> 4) & 0x0F0F0F0Fu) | ((hd[2] >> 2) & 0x30303030u);
+              u32x4 mw;
+              mw[0] = as_u((as_h2((mnl & kB02) | kMagic) - k1024) * k32);
+              mw[1] = as_u((as_h2(((mnl >> 8) & kB02) | kMagic) - k1024) * k32);
+              mw[2] = as_u((as_h2((mnh & kB02) | kMagic) - k1024) * k32);
+              mw[3] = as_u((as_h2(((mnh >> 8) & kB02) | kMagic) - k1024) * k32);
+    #pragma unroll
+              for (int i = 0; i < TT; ++i) {
+                f32x16 mt;
+    #pragma unroll
+                for (int e = 0; e < 16; ++e) mt[e] = 0.f;
+                mt = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, Hb[(NW + i) * 64 + al]),
+                                                            __builtin_bit_cast(f16x8, mw), mt, 0, 0, 0);
+    #pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                  if constexpr (decltype(fine)::value)
+                    acc[i][e] = fmaf(d, (tmp[i][0][e] + tmp[i][1][e]) * bs[e % NV], fmaf(-dm, mt[e] * bs[e % NV], acc[i][e]));
+                  else
+                    acc[i][e] = fmaf(d, tmp[i][0][e] + tmp[i][1][e], fmaf(-dm, mt[e], acc[i][e]));
+                }
+              }
+            }
+          } else {
+            // Q6_K: group g = K16 slice g. With q = n + 16 b (nibble n, qh field b), sc_g (q - 32) / 4 is the
+            // sum of two operands that f16 holds exactly, sc_g n / 4 (up to 480) and 4 sc_g (b - 2) (up to
+            // 1024), each one fma of the field under the exponent of 1024 (n 2^(4 c), b 2^(6 + 2 hi)). Both
+            // feed one chain, whose running sum is that of the whole weights: with a chain each the error
+            // against 64 bits is 4% larger.
+            const uint2 *Q = reinterpret_cast<const uint2 *>(Sb);
+            const u32x4 hd = Hb[hl];
 #pragma unroll
-            for (int i = 0; i < TT; ++i)
+            for (int c = 0; c < 2; ++c) {
+              const uint32_t sw = hd[2 * hh + c] ^ k80;
 #pragma unroll
-              for (int e = 0; e < 16; ++e) acc[i][e] = fmaf(d, tmp[i][0][e] + tmp[i][1][e], acc[i][e]);
+              for (int h = 0; h < 2; ++h) {
+                const h2 P = as_h2(((h ? sw >> 8 : sw) & kB02) | kMagic) - k1152;  // scales of hi = 0, 1
+                const h2 SP = P * (c ? k64th : k4th), NP = SP * kN1024, TP = P * kTb, OP = P * kOb;
+                const uint2 qa = Q[ql + 32 * h], qb = Q[ql + 64 + 32 * h], qh = Q[qq + 32 * h];
+#pragma unroll
+                for (int hi = 0; hi < 2; ++hi) {
+                  const _Float16 s = hi ? SP.y : SP.x, n = hi ? NP.y : NP.x, t = hi ? TP.y : TP.x, o = hi ? OP.y : OP.x;
+                  const h2 S = {s, s}, N0 = {n, n}, T = {t, t}, O = {o, o};
+                  const uint32_t mn = c ? kHi : kLo, mb = hi ? kB8 : kB6;
+                  u32x4 vn, vb;
+#pragma unroll
+                  for (int m = 0; m < 2; ++m) {
+                    const uint32_t x = hi ? (m ? qb.y : qb.x) : (m ? qa.y : qa.x), b4 = m ? qh.y : qh.x;
+                    const uint32_t be = b4 << (c ? 2 : 6), bo = b4 >> (c ? 6 : 2);
+                    vn[2 * m] = as_u(__builtin_elementwise_fma(as_h2((x & mn) | kMagic), S, N0));
+                    vn[2 * m + 1] = as_u(__builtin_elementwise_fma(as_h2(((x >> 8) & mn) | kMagic), S, N0));
+                    vb[2 * m] = as_u(__builtin_elementwise_fma(as_h2((be & mb) | kMagic), T, O));
+                    vb[2 * m + 1] = as_u(__builtin_elementwise_fma(as_h2((bo & mb) | kMagic), T, O));
+                  }
+#pragma unroll
+                  for (int i = 0; i < TT; ++i) {
+                    const f16x8 a = __builtin_bit_cast(f16x8, Sb[(i * 8 + 4 * c + 2 * hi + h) * 64 + al]);
+                    f32x16 z = tmp[i][hi];
+                    if (hh == 0 && c == 0 && h == 0)
+#pragma unroll
+                      for (int e = 0; e < 16; ++e) z[e] = 0.f;
+                    z = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, __builtin_bit_cast(f16x8, vn), z, 0, 0, 0);
+                    tmp[i][hi] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, __builtin_bit_cast(f16x8, vb), z, 0, 0, 0);
+                  }
+                }
+              }
+            }
+            if (hh == 1) {
+              const float d = 4.f * (float)reinterpret_cast<const _Float16 *>(Hb)[dl];
+#pragma unroll
+              for (int i = 0; i < TT; ++i)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                  if constexpr (decltype(fine)::value)
+                    acc[i][e] = fmaf(d, (tmp[i][0][e] + tmp[i][1][e]) * bs[e % NV], acc[i][e]);
+                  else
+                    acc[i][e] = fmaf(d, tmp[i][0][e] + tmp[i][1][e], acc[i][e]);
+                }
+            }
           }
         }
+        if (hh == 0)
+          FHIP_LDS_BARRIER_MID(wait_vm_mid(kEven));
+        else
+          FHIP_LDS_BARRIER_MID(wait_vm_mid(kOdd));
       }
-      if (hh == 0)
-        FHIP_LDS_BARRIER_MID(wait_vm_mid(kEven));
-      else
-        FHIP_LDS_BARRIER_MID(wait_vm_mid(kOdd));
     }
-  }
+  };
+  // In a loop of its own; two operand tiles have none (more than 32 tokens).
+  if (TT == 1 && __builtin_amdgcn_ballot_w64(tsl < 0.f) != 0)
+    range(std::integral_constant<bool, TT == 1>{});
+  else
+    range(std::false_type{});
   __builtin_amdgcn_s_waitcnt(wait_vm_mid(0));
 
   const int o = 32 * NW * ng + 32 * wave + rho;
   if (o >= N) return;
-  constexpr int TPT = HL ? 16 : 32, NV = HL ? 8 : 16;
   float4 sc[TT][NV / 4];  // every scale before the first store: a store would wait for a load after it
 #pragma unroll
   for (int i = 0; i < TT; ++i)
@@ -365,7 +428,7 @@ __global__ __launch_bounds__(64 * NW) void quant_mid_kernel(const uint8_t *__res
       const int tok = TPT * (TT * mg + i) + 8 * (e >> 2) + 4 * kap + (e & 3);
       if (tok >= M) continue;
       const float v = (HL ? acc[i][e] + acc[i][(e + 8) & 15] : acc[i][e]) *
-                      ((e & 3) == 0 ? sc[i][e >> 2].x : (e & 3) == 1 ? sc[i][e >> 2].y : (e & 3) == 2 ? sc[i][e >> 2].z : sc[i][e >> 2].w);
+                      fabsf((e & 3) == 0 ? sc[i][e >> 2].x : (e & 3) == 1 ? sc[i][e >> 2].y : (e & 3) == 2 ? sc[i][e >> 2].z : sc[i][e >> 2].w);
       if (SK == 1)
         Y[(size_t)tok * N + o] = v;
       else
@@ -387,7 +450,7 @@ constexpr size_t kMidScratch = (size_t)48 << 20;
 struct MidPlan {
   bool hl;
   int TT, NW, MTG, tokens, tasks, SK;
-  size_t xb, tb, pb;  // operands, token scales, K-range partial results
+  size_t xb, tb, bb, pb;  // operands, token scales, super-block scales, K-range partial results
   float cost;
 };
 
@@ -428,6 +491,7 @@ MidPlan plan_mid(int fmt, int N, int K, int M, int TT, int NW) {
     if (rounds > 3.f) break;  // more ranges only add rounds
   }
   p.tb = ((size_t)p.SK * p.tokens * 4 + 255) & ~(size_t)255;
+  p.bb = M <= 32 ? ((size_t)p.tokens * nblk * 4 + 255) & ~(size_t)255 : 0;
   p.pb = p.SK > 1 ? (size_t)p.SK * M * N * 4 : 0;
   return p;
 }
@@ -482,7 +546,7 @@ bool q6k_mid_takes(int N, int K, int M) {
 
 size_t mid_ws_bytes(int fmt, int N, int K, int M) {
   const MidPlan p = plan_mid(fmt, N, K, M);
-  return p.xb + p.tb + p.pb;
+  return p.xb + p.tb + p.bb + p.pb;
 }
 
 namespace {
@@ -490,22 +554,22 @@ template <int FMT>
 int launch_mid(const void *Wv, const float *X, float *Y, int N, int K, int M) {
   const MidPlan p = plan_mid(FMT, N, K, M);
   const int nblk = K / 256, ntiles = q4k_tiles(N), SK = p.SK, MTG = p.MTG, tokens = p.tokens;
-  const size_t xb = p.xb, tb = p.tb, pb = p.pb;
-  unsigned char *ws = (unsigned char *)workspace(xb + tb + pb);
+  const size_t xb = p.xb, tb = p.tb, bb = p.bb, bytes = xb + tb + bb + p.pb;
+  unsigned char *ws = (unsigned char *)workspace(bytes);
   if (!ws) return FHIP_ENOMEM;
-  if (int rc = check_disjoint("quant_mid", X, (size_t)M * K * 4, ws, xb + tb + pb)) return rc;
+  if (int rc = check_disjoint("quant_mid", X, (size_t)M * K * 4, ws, bytes)) return rc;
   u32x4 *xa = (u32x4 *)ws;
-  float *ts = (float *)(ws + xb), *part = (float *)(ws + xb + tb);
+  float *ts = (float *)(ws + xb), *bs = bb ? (float *)(ws + xb + tb) : nullptr, *part = (float *)(ws + xb + tb + bb);
   const dim3 pg(tokens, SK);
   const int units = 32 * ceil_div(nblk, SK);
   auto prep = [&](auto hl) {
     constexpr bool H = decltype(hl)::value;
     if (units <= 256)
-      mid_xprep_kernel<H, 1><<<pg, 256, 0, stream()>>>(X, M, K, nblk, SK, xa, ts);
+      mid_xprep_kernel<H, 1><<<pg, 256, 0, stream()>>>(X, M, K, nblk, SK, xa, ts, bs);
     else if (units <= 512)
-      mid_xprep_kernel<H, 2><<<pg, 256, 0, stream()>>>(X, M, K, nblk, SK, xa, ts);
+      mid_xprep_kernel<H, 2><<<pg, 256, 0, stream()>>>(X, M, K, nblk, SK, xa, ts, bs);
     else
-      mid_xprep_kernel<H, 0><<<pg, 256, 0, stream()>>>(X, M, K, nblk, SK, xa, ts);
+      mid_xprep_kernel<H, 0><<<pg, 256, 0, stream()>>>(X, M, K, nblk, SK, xa, ts, bs);
   };
   if (p.hl)
     prep(std::true_type{});
@@ -514,7 +578,7 @@ int launch_mid(const void *Wv, const float *X, float *Y, int N, int K, int M) {
   FHIP_CHECK_LAUNCH("mid_xprep_kernel");
   const uint8_t *W = (const uint8_t *)Wv;
   auto run = [&](auto kern) {
-    kern<<<p.tasks * SK, 64 * p.NW, 0, stream()>>>(W, xa, ts, Y, part, N, M, nblk, ntiles, MTG, tokens, SK);
+    kern<<<p.tasks * SK, 64 * p.NW, 0, stream()>>>(W, xa, ts, bs, Y, part, N, M, nblk, ntiles, MTG, tokens, SK);
   };
   if (p.hl)
     run(quant_mid_kernel<FMT, 1, true, 4>);
