@@ -478,14 +478,16 @@ extern "C" int fhip_q4k_matmul_int8_f32(const void *dPacked, const float *dX, fl
   const int ntiles = q4k_tiles(out);
   // One token, except on the widest matrices' long rows, whose parked terms leave a CU too few waves
   // where the general kernel's eight-tile workgroups park none (us, one-token / general: 25600 x 4096
-  // 17.8 / 18.4, 25600 x 5120 23.0 / 20.9, 152064 x 3584 63.9 / 87.4, 152064 x 5120 127 / 101, 16384 x
-  // 11008 57 / 40).
+  // 17.8 / 18.4, 25600 x 5120 23.0 / 20.9, 152064 x 3584 63.9 / 87.4, 152064 x 5120 127 / 101). At four
+  // tiles per CU both change shape: the one-token kernel's waves per tile halve, the general kernel's
+  // workgroups take eight tiles (16368 x 11008 31.0 / 44.6, 16384 x 11008 57 / 40; 16368 x 4352 14.1 / 27.3).
+  // Below, the one-token kernel took 0.47 to 0.94 of the general one's time at 267 shapes of 64 to 1023 tiles by 6
+  // to 100 super-blocks (1024 x 6144 9.5 / 10.1, 12800 x 11008 29 / 41, 10240 x 25600 64 / 117).
   if (P == 1 && tuning().i8r_kw <= 0 && tuning().i8r_tw <= 0 && (ntiles < 4 * cu_count() || nblk <= 16) &&
       i8r1_lds(nblk, 1) <= (size_t)lds_limit()) {
     // Waves per tile until the grid has eight per CU (each at least a record) and the workgroups that fit
-    // a CU's LDS have twelve, then tiles per workgroup,
-    // which share its quantized activation, up to four waves while the grid covers the CUs twice and
-    // two workgroups' terms fit in LDS. us at waves x tiles: 18944 x 3584 2 x 2 12.8, 4 x 1 14.1, 4 x 2
+    // a CU's LDS have twelve, then tiles per workgroup, which share its quantized activation, up to four
+    // waves while the grid covers the CUs twice and two workgroups' terms fit in LDS. us at waves x tiles: 18944 x 3584 2 x 2 12.8, 4 x 1 14.1, 4 x 2
     // 16.4, 1 x 4 13.8; 152064 x 3584 1 x 4 64, 2 x 2 65, 4 x 1 83; 3584 x 18944 16 x 1 18.2, 8 x 1 20.0.
     const int cus = cu_count() > 0 ? cu_count() : 256;
     int KW = 1, TW = 1;

@@ -1,7 +1,8 @@
 """The int8 route's one-token kernel (q4k_i8route1_kernel) at the edges of its shapes, bit for bit
 against the oracle: rows around a 16-row tile, fewer records than waves, a wave split of every size,
 several tiles per workgroup, rows longer than the activations a workgroup holds in registers, the
-longest row whose terms fit in LDS and one past it (the general kernel), zero, subnormal and
+longest row whose terms fit in LDS and one past it (the general kernel), the last tile count it takes on
+long rows and the next, zero, subnormal and
 non-finite activation blocks."""
 import numpy as np
 import pytest
@@ -15,7 +16,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("out,in_", [(1, 256), (15, 512), (17, 768), (100, 3584), (520, 4352),
                                      (8200, 256), (16500, 1280), (48, 18944), (33, 30976),
-                                     (33, 31232)])
+                                     (33, 31232), (16368, 4352), (16384, 4352)])
 def test_shapes(hip, oracle_mod, out, in_):
     print(f"[case] int8 one token out={out} in={in_}", flush=True)
     raw = synth.q4k_weights(out, in_, out + in_)
