@@ -185,3 +185,72 @@ def test_graph_decode_ffn_replays(hip):
         for p in allocs:
             lib.fhip_free(p)
         fakhip.call("fhip_stream_destroy", st)
+
+
+def test_graph_batched_routes(hip):
+    """The wider routes captured: prefill GEMMs of Q4_K (all tiles in K ranges, and a tail of them) and
+    Q6_K, the staged few-token kernel (hi and lo rows, f16 rows, two operand tiles), the Q8_0 GEMM (one and
+    two token tiles per workgroup) and the one-token int8 kernel. Four replays give the bits of the same
+    calls run eagerly between them, on ordinary activations and on ones whose ranges need block scales."""
+    from tests import q6k_cases as qc
+    lib = fakhip.load()
+    st = C.c_void_p()
+    fakhip.call("fhip_stream_create", C.byref(st))
+    fakhip.call("fhip_set_stream", st)
+    ws, devs = {}, []
+    rng = np.random.default_rng(9)
+    #        name: entry, weight's format, out, in, P
+    calls = {"gemm": ("fhip_q4k_matmul_f32", "q4k", 1024, 4096, 140),
+             "gemm tail": ("fhip_q4k_matmul_f32", "q4k", 33024, 1024, 129),
+             "gemm q6k": ("fhip_q6k_matmul_f32", "q6k", 520, 2048, 140),
+             "mid hi lo": ("fhip_q4k_matmul_f32", "q4k", 1024, 4096, 9),
+             "mid f16": ("fhip_q6k_matmul_f32", "q6k", 520, 2048, 24),
+             "mid two tiles": ("fhip_q4k_matmul_f32", "q4k", 33024, 1024, 50),
+             "gemm q8_0": ("fhip_q8_0_matmul_f32", "q8_0", 300, 2080, 40),
+             "gemm q8_0 two": ("fhip_q8_0_matmul_f32", "q8_0", 2100, 4096, 150),
+             "int8": ("fhip_q4k_matmul_int8_f32", "q4k", 1024, 4096, 1)}
+    try:
+        for name, (entry, fmt, out, in_, P) in calls.items():
+            raw = (synth.q4k_weights(out, in_, 3) if fmt == "q4k" else synth.q8_0_weights(out, in_, 4) if fmt == "q8_0"
+                   else qc.pin_d(rng.integers(0, 256, out * (in_ // 256) * 210, dtype=np.uint8), 0x1400))
+            ws[name] = fakhip.alloc_call("fhip_%s_upload" % fmt, raw.ctypes.data, out, in_)
+        x = Dev(150 * 4096 * 4)
+        devs.append(x)
+        ys = {name: (Dev(c[4] * c[2] * 4), Dev(c[4] * c[2] * 4)) for name, c in calls.items()}
+        devs += [d for pair in ys.values() for d in pair]
+
+        def run(k):
+            for name, (entry, fmt, out, in_, P) in calls.items():
+                fakhip.call(entry, ws[name], x.ptr, ys[name][k].ptr, out, in_, P)
+
+        def set_x(seed, far):
+            a = synth.activations(150, 4096, seed)
+            if far:
+                a.reshape(-1)[::700] *= np.float32(1e7)
+            fakhip.call("fhip_h2d", x.ptr, a.ctypes.data, a.nbytes)
+
+        set_x(1, False)
+        run(0)  # eager warm-up: sizes the workspace before capture
+        fakhip.call("fhip_sync")
+        fakhip.call("fhip_graph_begin")
+        run(0)
+        graph = C.c_void_p()
+        fakhip.call("fhip_graph_end", C.byref(graph))
+        try:
+            for rep in range(4):
+                set_x(10 + rep, rep % 2 == 1)
+                run(1)
+                fakhip.call("fhip_graph_launch", graph)
+                fakhip.call("fhip_stream_sync", st)
+                for name, (a, b) in ys.items():
+                    assert np.array_equal(a.to_host(np.uint32), b.to_host(np.uint32)), (rep, name)
+                print(f"    replay {rep}: all {len(ys)} outputs bit-identical", flush=True)
+        finally:
+            fakhip.call("fhip_graph_destroy", graph)
+    finally:
+        fakhip.call("fhip_set_stream", None)
+        for d in devs:
+            d.close()
+        for p in ws.values():
+            lib.fhip_free(p)
+        fakhip.call("fhip_stream_destroy", st)

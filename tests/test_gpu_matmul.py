@@ -2,7 +2,7 @@
 inputs, at the reference's tolerances (metric of internal/model/quant_q4k_test.go:140-158):
 
   GEMV (P <= 16, f32-accumulate)  max|dY|/RMS(Y_ref) <= 1e-3
-  P > 16 (f16 MFMA: 17..32 on the small-M kernel's f16 form, more on the prefill GEMM)
+  P > 16 (f16 MFMA: a few tens of tokens on the staged kernel, more on the prefill GEMM)
                                   max|dY|/RMS(Y_ref) <= 1e-2
 
 Shapes: the five workloads (Q8_0 576->1536; Q4_K 3584->18944 and 18944->3584; prefill
@@ -46,7 +46,9 @@ def _check_q4k(oracle_mod, out, in_, P, seed, tol, workers=16, rows=None):
 
 @pytest.mark.parametrize("out,in_,P", [
     (16, 256, 1), (1, 256, 1), (9, 512, 1), (33, 768, 3), (320, 256, 8), (100, 1024, 16),
-    (64, 2560, 5), (17, 4096, 13)])
+    (64, 2560, 5), (17, 4096, 13),
+    # few rows of more than 24576 values: quant_gemv16_kernel, ragged rows, a last range padded to a pair
+    (1001, 24832, 5), (517, 24832, 16), (33, 26112, 11)])
 def test_q4k_gemv_small_shapes(hip, oracle_mod, out, in_, P):
     _check_q4k(oracle_mod, out, in_, P, seed=out * 31 + in_ + P, tol=GEMV_TOL)
 
@@ -93,10 +95,11 @@ def test_q4k_gemv_global_operands_forced(hip, oracle_mod, monkeypatch, out, in_,
     assert np.array_equal(lds.view(np.uint32), glob.view(np.uint32))
 
 
-def test_q4k_gemv16_from_knob_is_clamped(hip, oracle_mod, monkeypatch):
+@pytest.mark.parametrize("out,in_,P", [(512, 2048, 6), (512, 24832, 6)])
+def test_q4k_gemv16_from_knob_is_clamped(hip, oracle_mod, monkeypatch, out, in_, P):
     """FAK_HIP_GEMV16_FROM names the first width on the 5..16-token kernel; values the int8
-    kernel cannot take (it holds 1..4 tokens) are ignored, so 6 tokens still get every row."""
-    out, in_, P = 512, 2048, 6
+    kernel cannot take (it holds 1..4 tokens) are ignored, so 6 tokens still get every row. (The
+    second shape is one that the staged kernel leaves to the choice.)"""
     raw = synth.q4k_weights(out, in_, seed=66)
     X = synth.activations(P, in_, seed=67)
     with knobs(monkeypatch, FAK_HIP_GEMV16_FROM=8):
@@ -202,7 +205,10 @@ def test_q4k_small_m_27b(hip, oracle_mod, out, in_, P):
 
 
 @pytest.mark.parametrize("out,in_,P", [(256, 512, 33), (300, 768, 40), (512, 1024, 128),
-                                       (1000, 2048, 200), (64, 256, 1000)])
+                                       (1000, 2048, 200), (64, 256, 1000),
+                                       # one partial token tile on the GEMM: more than 12288 rows
+                                       (12301, 1024, 65), (12301, 512, 77), (12301, 768, 127),
+                                       (12301, 256, 128)])
 def test_q4k_gemm_small_shapes(hip, oracle_mod, out, in_, P):
     _check_q4k(oracle_mod, out, in_, P, seed=out + in_ + P, tol=GEMM_TOL)
 
@@ -211,8 +217,8 @@ def test_q4k_gemm_small_shapes(hip, oracle_mod, out, in_, P):
                                        (5120, 25600, 20), (1000, 2048, 19), (300, 768, 32),
                                        (16, 256, 31), (100, 1024, 25)])
 def test_q4k_small_prefill_17_to_32(hip, oracle_mod, out, in_, P):
-    """17..32 tokens on the 32x32 small-M kernel with one f16 operand row per token (K split in
-    ranges at the long shapes): every output against the oracle at the GEMM bound."""
+    """17..32 tokens on the staged kernel with one f16 operand row per token (K split in ranges at
+    the long shapes): every output against the oracle at the GEMM bound."""
     rows = 256 if out * in_ > 4096 * 4096 else None
     e = _check_q4k(oracle_mod, out, in_, P, seed=3 * out + in_ + P, tol=GEMM_TOL, rows=rows)
     assert e <= 2e-3, e  # f16 activations under a per-token power-of-two scale: ~1e-3
@@ -293,7 +299,8 @@ def test_q4k_gemm_wide_tiles(hip, oracle_mod, monkeypatch, out, in_, P):
 
 
 @pytest.mark.parametrize("out,in_,P", [(3584, 18944, 512), (1000, 2048, 520), (18944, 3584, 128),
-                                       (300, 4096, 40), (3584, 18944, 1024), (3000, 18944, 1000)])
+                                       (300, 4096, 40), (3584, 18944, 1024), (3000, 18944, 1000),
+                                       (300, 4096, 140), (13001, 4096, 77)])
 def test_q4k_gemm_k_split(hip, oracle_mod, out, in_, P):
     """Grids too small for the GPU split K and add the ranges' partial sums in range order: the
     result meets the GEMM bound against the oracle (sampled rows for the 7B shapes) and is the

@@ -1,7 +1,7 @@
-"""The Q4_K kernel for a few tokens to a few tens (q4k_mid_kernel) at the edges of its tiles: rows
-around a workgroup's 128 or 256, one super-block to ranges that are no multiple of its three-stage
-passes, every operand form (hi and lo rows up to 16 tokens, one or two tiles of 32 above, several
-groups of tokens), against the weights dequantized on the host in 64 bits.
+"""The Q4_K kernel for a few tokens to a few tens (quant_mid_kernel) at the edges of its tiles: rows
+around a workgroup's 128, one super-block to ranges that are no multiple of its three-stage passes,
+hi and lo rows up to 16 tokens, tiles of 32 above, several groups of tokens, against the weights
+dequantized on the host in 64 bits. (Two operand tiles, 256 rows: test_gpu_mid_forms.py.)
 
 Tolerances, max|d|/RMS: up to 16 tokens an activation carries 22 bits below its range's largest
 magnitude and every product is exact, so the error is a few 2^-22: 1e-5. Above, activations are f16
@@ -11,7 +11,8 @@ import numpy as np
 import pytest
 
 from fak_amd import synth
-from tests.gpu_util import Dev, q4k_matmul, q4k_matmul_group, rel_err_rows, scaled_activations
+from tests.gpu_util import (Dev, q4k_matmul, q4k_matmul_group, rel_err_rows, scaled_activations,
+                            spread_rows)
 
 pytestmark = pytest.mark.gpu
 
@@ -73,7 +74,8 @@ def test_group_members(hip):
 
 @pytest.mark.parametrize("out,in_,P", [(78848, 2560, 64), (2048, 65536, 64), (40, 262144, 32)])
 def test_scratch_stays_small(hip, out, in_, P):
-    """Operands and partial results fit the no-allocation entry's 64 MiB at tall and at long weights."""
+    """Operands and partial results fit the no-allocation entry's 64 MiB at tall and at long weights; both
+    entries give the same bits, right on rows of every 128."""
     lib = hip.load()
     print(f"[case] q4k mid scratch out={out} in={in_} P={P}", flush=True)
     raw = synth.q4k_weights(out, in_, seed=1)
@@ -85,5 +87,8 @@ def test_scratch_stays_small(hip, out, in_, P):
             Y = dy.to_host(np.float32).reshape(P, out)
             hip.call("fhip_q4k_matmul_f32", w, dx.ptr, dy.ptr, out, in_, P)
             np.testing.assert_array_equal(Y, dy.to_host(np.float32).reshape(P, out))
+            rows = spread_rows(out, per_block=1)
+            sub = raw.reshape(out, -1)[rows].reshape(-1)
+            assert rel_err_rows(Y[:, rows], exact(sub, len(rows), in_, X)) <= tol(P)
     finally:
         lib.fhip_free(w)

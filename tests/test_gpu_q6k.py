@@ -63,7 +63,8 @@ def test_gemv_reference_fixture_exact(hip, oracle_mod):
                                        (4096, 512, 3), (37, 256, 8), (17, 66048, 1),
                                        (152064, 3584, 1), (3584, 18944, 2), (3584, 18944, 16),
                                        (1000, 2048, 13), (300, 768, 16), (18944, 3584, 1),
-                                       (5120, 4096, 1), (14336, 1024, 1), (8192, 768, 1)])
+                                       (5120, 4096, 1), (14336, 1024, 1), (8192, 768, 1),
+                                       (1001, 24832, 2), (517, 24832, 16), (33, 26112, 5)])
 def test_gemv_matches_oracle(hip, oracle_mod, out, in_, P):
     print(f"[case] q6k gemv out={out} in={in_} P={P}", flush=True)
     rng = np.random.default_rng(out + in_ + P)
@@ -132,8 +133,8 @@ def test_argument_errors(hip):
                                             (3584, 18944, 128, 48), (3584, 18944, 1024, 48),
                                             (3000, 18944, 1000, 48), (18944, 3584, 1024, 64)])
 def test_gemm_prefill_matches_oracle(hip, oracle_mod, out, in_, P, rows):
-    """More than 16 tokens (17..32 on the small-M kernel's f16 form, more on the f16 MFMA prefill
-    GEMM, its 256-row workgroups with K ranges from eight token tiles on the long rows) on the
+    """More than 16 tokens (a few tens, 128 on a small matrix, on the staged kernel, more on the f16 MFMA
+    prefill GEMM, its 256-row workgroups with K ranges from eight token tiles on the long rows) on the
     Q6_K records: max|dY|/RMS <= 1e-2 (the GEMM bound), checked on every output or on a sample
     of rows at full shape."""
     print(f"[case] q6k gemm out={out} in={in_} P={P}", flush=True)
@@ -155,7 +156,8 @@ def test_gemm_prefill_matches_oracle(hip, oracle_mod, out, in_, P, rows):
 
 
 @pytest.mark.parametrize("out,in_,P", [(300, 768, 40), (1000, 2048, 200), (152, 4096, 131),
-                                       (3584, 18944, 128), (18944, 3584, 512)])
+                                       (3584, 18944, 128), (18944, 3584, 512), (300, 768, 140),
+                                       (16500, 1280, 77)])
 def test_gemm_forms_bit_identical(hip, oracle_mod, monkeypatch, out, in_, P):
     """The staged prefill GEMM (the default: weights loaded straight to the registers of the
     lanes that use them) and the four-wave 2x2 form (records staged through LDS) share the tile,

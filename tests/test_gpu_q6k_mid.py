@@ -1,7 +1,8 @@
 """The Q6_K kernel for a few tokens to a few tens (quant_mid_kernel) at the edges of its tiles: rows around
-a workgroup's 128 or 256, one super-block to ranges that are no multiple of its three-stage passes, grids
-that the 8 XCDs divide unevenly, every operand form (hi and lo rows up to 16 tokens, one or two tiles of
-32 above, several groups of tokens), against the weights decoded from the layout, summed in 64 bits.
+a workgroup's 128, one super-block to ranges that are no multiple of its three-stage passes, grids that
+the 8 XCDs divide unevenly, hi and lo rows up to 16 tokens, tiles of 32 above, several groups of tokens,
+against the weights decoded from the layout, summed in 64 bits. (Two operand tiles, 256 rows:
+test_gpu_mid_forms.py.)
 
 Tolerances, max|d|/RMS: up to 16 tokens an activation carries 22 bits below its range's largest magnitude
 and every weight operand is exact, so the error is a few 2^-22: 1e-5. Above, activations are f16 (2^-11

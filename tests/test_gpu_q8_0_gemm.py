@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from fak_amd import synth
-from tests.gpu_util import knobs, q8_0_matmul, rel_err_rows, scaled_activations
+from tests.gpu_util import knobs, q8_0_matmul, rel_err_rows, scaled_activations, spread_rows
 
 pytestmark = pytest.mark.gpu
 
@@ -30,6 +30,23 @@ def test_shapes(hip, out, in_, P):
     raw = synth.q8_0_weights(out, in_, seed=out + in_)
     X = synth.activations(P, in_, P)
     assert rel_err_rows(q8_0_matmul(raw, out, in_, X, P), exact(raw, out, in_, X)) <= 1e-5
+
+
+@pytest.mark.parametrize("out,in_,P", [
+    # ranges of 33, 65 and 129 pairs of blocks (two, four units per thread of the operand launch, and a range
+    # read twice), the last half padding, K unsplit; one token tile per workgroup, then two
+    (2001, 2080, 510), (2001, 4128, 500), (1001, 8224, 1020), (4040, 2080, 500), (3601, 4128, 515),
+    (3601, 8224, 520),
+    # the same, K in ranges: the 7B shapes, and odd counts of blocks
+    (18944, 3584, 512), (2048, 18944, 512), (3584, 18944, 512), (2100, 5152, 150), (700, 19008, 1024)])
+def test_range_lengths(hip, out, in_, P):
+    print(f"[case] q8_0 gemm ranges out={out} in={in_} P={P}", flush=True)
+    rows = spread_rows(out)
+    raw = synth.q8_0_weights(out, in_, seed=out + in_)
+    X = synth.activations(P, in_, P)
+    Y = q8_0_matmul(raw, out, in_, X, P)
+    sub = raw.reshape(out, -1)[rows].reshape(-1)
+    assert rel_err_rows(Y[:, rows], exact(sub, len(rows), in_, X)) <= 1e-5
 
 
 @pytest.mark.parametrize("pattern", ["all", "wee"])

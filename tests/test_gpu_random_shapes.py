@@ -1,6 +1,6 @@
 """Seeded random shapes across every route of the Q4_K and Q6_K matmuls (the 1..4-token int8
-GEMV, the 5..16-token kernel, its 17..32-token f16 form, the prefill GEMM on 128- and 256-row
-workgroups with and without K ranges), each against the oracle at its bound: max|dY|/RMS <= 1e-3
+GEMV, the 5..16-token kernel, the staged kernel for a few to a few tens, the prefill GEMM on 128- and
+256-row workgroups with and without K ranges), each against the oracle at its bound: max|dY|/RMS <= 1e-3
 up to 16 tokens, 1e-2 beyond. Activations are N(0,1) times a per-case power of ten in
 [1e-3, 1e3]; outputs are checked on every row, or on rows spread over every row block for the
 largest products."""

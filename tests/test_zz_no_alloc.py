@@ -18,11 +18,10 @@ def run(fn, w, X, out, in_, P):
 
 
 # (out, in, P): a K-split prefill GEMM (operands + token scales + partials: ~56 MB of scratch),
-# then smaller calls: a 16-token GEMV with K-range partials, a 3-token GEMV with global
-# activation operands, one decode token, a 24-token call (the 17..32-token route, K-range
-# partials sized for its tokens), a 4-token call at in >= 24576 (which takes the 5..16-token
-# kernel's route from three tokens) and a 1024-token GEMM on 256-row workgroups in 4 K ranges
-# (~52 MB of scratch).
+# then smaller calls: 16 and 24 tokens on the staged kernel (its operands, and K-range partials sized
+# for the tokens), a 3-token GEMV with global activation operands, one decode token, a 4-token call at
+# in >= 24576 (which takes the 5..16-token kernel's route from three tokens) and a 1024-token GEMM on
+# 256-row workgroups in 4 K ranges (~52 MB of scratch).
 CALLS = [(3584, 18944, 512), (2048, 6144, 16), (3584, 18944, 3), (1024, 3584, 1),
          (18944, 3584, 24), (5120, 25600, 4), (3584, 4096, 1024)]
 
