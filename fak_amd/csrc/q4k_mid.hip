@@ -16,14 +16,14 @@
 // in the loop. What bounds it: a workgroup's super-block takes about 1.15 us (Q6_K 1.6: a wave's own
 // chain of LDS reads, unpack and MFMAs; its 37 (44) KB of direct loads hide behind it), two on a CU
 // 1.7 (2.5), near the memory's pace; so time is the longest range, plus the launches before and after it.
-// us per call against the kernels it replaced (q4k_gemv16.hip, up to 16 tokens and its former 32-token
-// form up to 32, the prefill GEMM for more):
-//   Q4_K 3584 x 3584 at 8 / 16 / 32 / 64 tokens   18.1 / 18.6 / 18.2 / 22.8 -> 10.7 / 11.4 / 12.7 / 15.1
-//        18944 x 3584                             19.3 / 20.7 / 29.0 / 31.3 -> 17.7 / 18.6 / 20.1 / 25.9
-//        8192 x 11008                             28.0 / 29.5 / 39.3 / 37.3 -> 19.3 / 21.5 / 21.9 / 29.0
-//   Q6_K 3584 x 3584 at 2 / 16 / 32 / 64          18.2 / 18.8 / 21.5 / 23.2 -> 11.6 / 13.1 / 14.1 / 17.1
-//        18944 x 3584                             26.1 / 28.0 / 34.7 / 35.3 -> 21.2 / 23.0 / 24.5 / 32.0
-//        5120 x 25600                             41.8 / 45.6 / 55.2 / 58.2 -> 35.7 / 37.8 / 39.2 / 50.6
+// us per call with cold weights (9 to 16 copies in turn) against the kernels it replaced (q4k_gemv16.hip, up
+// to 16 tokens and its former 32-token form up to 32, the prefill GEMM for more):
+//   Q4_K 3584 x 3584 at 8 / 16 / 32 / 64 tokens   18.1 / 18.5 / 18.2 / 22.4 -> 12.0 / 12.8 / 14.1 / 15.7
+//        18944 x 3584                             20.7 / 21.8 / 30.6 / 34.1 -> 20.4 / 21.7 / 23.2 / 31.1
+//        8192 x 11008                             31.2 / 33.4 / 42.5 / 41.0 -> 22.5 / 24.3 / 25.7 / 34.8
+//   Q6_K 3584 x 3584 at 2 / 16 / 32 / 64          18.1 / 18.7 / 21.3 / 26.0 -> 12.9 / 13.5 / 14.8 / 17.0
+//        18944 x 3584                             29.0 / 32.0 / 36.6 / 38.8 -> 24.0 / 27.8 / 29.2 / 36.8
+//        5120 x 25600                             42.5 / 47.7 / 55.8 / 60.9 -> 36.3 / 40.7 / 41.4 / 54.1
 #include <type_traits>
 
 #include "kernels.hpp"
