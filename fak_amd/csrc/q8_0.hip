@@ -258,19 +258,17 @@ __global__ void q8_xprep_kernel(const float *__restrict__ X, int K, int ns, int 
   split_slice<M>(X + (size_t)t * K + 32 * (sl < nsv ? sl : 0), sl < nsv, sl, t, A, E);
 }
 
-template <int M>
-bool q8_lds_x(int K) {
-  constexpr int VALS = ((2 * M + 15) / 16) * (M < 2 ? M : 2);
-  const size_t stage = xop_bytes(M, 2 * q8_groups(K));
-  return !tuning().gemv_globalx && stage + (size_t)16 * 64 * VALS * 4 <= (size_t)lds_limit();
-}
-
-template <int M>
-int launch_q8(const uint8_t *W, const float *X, float *Y, int N, int K) {
-  const int npairs = q8_groups(K), ntiles = q4k_tiles(N), ns = 2 * npairs;
-  constexpr int VALS = ((2 * M + 15) / 16) * (M < 2 ? M : 2);
-  const size_t stage = xop_bytes(M, ns);
-  const bool lds_x = q8_lds_x<M>(K);
+// Launch shape of the GEMV: tiles x K parts (waves) per workgroup, LDS bytes of the staged operands (0:
+// they stay in global memory) and of the split-K sum.
+struct Q8Shape {
+  int TW, KW, grid;
+  size_t stage, red;
+};
+Q8Shape q8_gemv_shape(int N, int K, int M) {
+  const int npairs = q8_groups(K), ntiles = q4k_tiles(N);
+  const size_t vals = (size_t)((2 * M + 15) / 16) * (M < 2 ? M : 2);  // per lane, for the split-K sum
+  const size_t stage = xop_bytes(M, 2 * npairs);
+  const bool lds_x = !tuning().gemv_globalx && stage + 16 * 64 * vals * 4 <= (size_t)lds_limit();
   const int max_waves = (lds_x && M <= 8) ? 16 : 8;
   int TW = tuning().q8_tw, KW = tuning().q8_kw;
   const int cus = cu_count() > 0 ? cu_count() : 256;
@@ -292,9 +290,16 @@ int launch_q8(const uint8_t *W, const float *X, float *Y, int N, int K) {
   if (TW <= 0) TW = max_waves / KW > 4 ? 4 : max_waves / KW;
   if (TW < 1) TW = 1;
   while (TW * KW > max_waves) TW--;
-  const int grid = ceil_div(ntiles, TW), threads = 64 * TW * KW;
-  const size_t redB = KW > 1 ? (size_t)TW * KW * 64 * VALS * 4 : 0;
-  if (lds_x) {
+  return Q8Shape{TW, KW, ceil_div(ntiles, TW), lds_x ? stage : 0, KW > 1 ? (size_t)TW * KW * 64 * vals * 4 : 0};
+}
+
+template <int M>
+int launch_q8(const uint8_t *W, const float *X, float *Y, int N, int K) {
+  const Q8Shape p = q8_gemv_shape(N, K, M);
+  const int npairs = q8_groups(K), ntiles = q4k_tiles(N), ns = 2 * npairs, TW = p.TW, KW = p.KW;
+  const int grid = p.grid, threads = 64 * TW * KW;
+  const size_t stage = xop_bytes(M, ns), redB = p.red;
+  if (p.stage) {
     // Measured (us, ring of 8 / ring of 1 before): 18944 x 3584 one token 21.6 / 23.2, 3584 x
     // 18944 four tokens 53.1 / 57.1; a 1536 x 576 matrix (about two records per wave) is
     // faster with the short ring.
@@ -323,13 +328,21 @@ int launch_q8(const uint8_t *W, const float *X, float *Y, int N, int K) {
 // in LDS is the shorter for a few tokens of a matrix up to a few tens of MB (us, GEMV / GEMM: 3584 x
 // 3584 at 8 tokens 9.3 / 12.1, 8192 x 2048 at 16 11.8 / 13.8, 2048 x 2048 at 16 9.1 / 10.6). The GEMM
 // is where the operands do not fit in LDS (3584 x 18944 at 2 tokens 49.9 / 23.2, 3584 x 3584 at 12
-// 17.4 / 12.4), from three tokens of a large matrix (18944 x 3584 at 2 / 4 / 8 tokens 22.7 / 21.5,
-// 23.9 / 21.7, 29.8 / 21.8) and above 16 tokens.
+// 17.4 / 12.4), above 16 tokens, above 8 of a large matrix, and from three tokens of a large matrix where
+// the GEMV's grid leaves CUs idle, with under 5/8 of what the fullest CU gets on average (18944 x 3584 at 2 / 4 /
+// 8 tokens 22.7 / 21.5, 23.9 / 21.7, 29.8 / 21.8; 16656 x 9600 at 3 64 / 50), or takes more than two rounds of
+// the workgroups that fit a CU's LDS (44640 x 3584 at 6 66 / 49). Elsewhere both run at memory's pace, and the
+// GEMM adds its two other launches (at 3 tokens 16208 x 6784 26.7 / 37.6, 39056 x 4096 39.2 / 53.8, 5200 x
+// 9600 20.1 / 22.6; two rounds, 31248 x 5120 at 4 40.7 / 47.6).
 bool q8_takes_gemv(int N, int K, int M) {
   if (M == 1 || (M <= 16 && tuning().gemv_globalx)) return true;
-  if (M > 16 || (M > 2 && (long long)N * K >= 32 << 20)) return false;
-  const size_t vals = (size_t)((2 * M + 15) / 16) * 2;  // per lane, for the split-K sum
-  return xop_bytes(M, 2 * q8_groups(K)) + 16 * 64 * vals * 4 <= (size_t)lds_limit();
+  if (M > 16) return false;
+  const Q8Shape p = q8_gemv_shape(N, K, M);
+  if (!p.stage) return false;
+  if (M == 2 || (long long)N * K < 32 << 20) return true;
+  const int cus = cu_count() > 0 ? cu_count() : 256, per = ceil_div(p.grid, cus);
+  const int fit = (int)((size_t)lds_limit() / (p.stage + p.red));  // >= 1
+  return M <= 8 && per <= 2 * fit && 8LL * p.grid >= 5LL * per * cus;
 }
 
 int check_q8_shape(const char *who, int out, int in) {

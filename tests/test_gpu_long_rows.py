@@ -111,10 +111,10 @@ def seconds(prefix, w, out, in_, P):
     with Dev(P * in_ * 4) as dx, Dev(P * out * 4) as dy:
         fakhip.call("fhip_memset_async", dx.ptr, 0, dx.nbytes)
         best = 1e9
-        for _ in range(5):
+        for _ in range(6):
             fakhip.call("fhip_sync")
             t = time.perf_counter()
-            for _ in range(4):
+            for _ in range(8):
                 fakhip.call(prefix + "_matmul_f32", w, dx.ptr, dy.ptr, out, in_, P)
             fakhip.call("fhip_sync")
             best = min(best, time.perf_counter() - t)

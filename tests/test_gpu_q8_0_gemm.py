@@ -49,6 +49,39 @@ def test_range_lengths(hip, out, in_, P):
     assert rel_err_rows(Y[:, rows], exact(sub, len(rows), in_, X)) <= 1e-5
 
 
+@pytest.mark.parametrize("out,in_,P", [(16208, 6784, 3), (16208, 6784, 5), (31248, 5120, 4), (30700, 3584, 6),
+                                       (39056, 4096, 5), (16650, 9600, 3), (33200, 1024, 8), (18944, 3584, 8),
+                                       (40000, 1056, 8), (40000, 1056, 9)])
+def test_few_tokens_of_a_large_matrix(hip, out, in_, P):
+    """Three to eight tokens of 32 M weights and more, on either side of the rule that picks the GEMV or the
+    GEMM, and nine. The GEMV's products of 1152 + code less 1152 times the sum round to a few 2^-20: 2e-5."""
+    print(f"[case] q8_0 few tokens out={out} in={in_} P={P}", flush=True)
+    rows = spread_rows(out)
+    few = synth.q8_0_weights(len(rows), in_, seed=out + in_)
+    raw = np.zeros((out, in_ // 32 * 34), np.uint8)
+    raw[rows] = few.reshape(len(rows), -1)
+    X = synth.activations(P, in_, P)
+    Y = q8_0_matmul(raw.reshape(-1), out, in_, X, P)
+    assert rel_err_rows(Y[:, rows], exact(few, len(rows), in_, X)) <= 2e-5
+    Y[:, rows] = 0
+    assert not Y.any()
+
+
+def test_three_tokens_cost_little_more_than_two(hip):
+    """Where both kernels run at memory's pace, the GEMM's three launches cost a third more than the GEMV's one."""
+    from tests.test_gpu_long_rows import seconds
+    out, in_ = 16208, 6784
+    print("[case] q8_0 time of 3 tokens against 2", flush=True)
+    lib = hip.load()
+    raw = np.zeros(out * (in_ // 32) * 34, np.uint8)
+    w = hip.alloc_call("fhip_q8_0_upload", raw.ctypes.data, out, in_)
+    try:
+        seconds("fhip_q8_0", w, out, in_, 3)
+        assert seconds("fhip_q8_0", w, out, in_, 3) < 1.25 * seconds("fhip_q8_0", w, out, in_, 2)
+    finally:
+        lib.fhip_free(w)
+
+
 @pytest.mark.parametrize("pattern", ["all", "wee"])
 def test_scales_and_special_values(hip, pattern):
     """Any finite activation scale, and a NaN or an infinity stays in its own token."""
