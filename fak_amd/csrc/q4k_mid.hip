@@ -539,8 +539,11 @@ bool q4k_mid_takes(int N, int K, int M) {
 // 17..32 tokens of more than a few rows of kF16Row to 2^20 values, whose two groups of 16 tokens read the
 // records through one L2 (us, q4k_gemv16.hip / this at 24 tokens: 3584 x 262400 524 / 377, 1000 x 262400
 // 156 / 132, 2000 x 524288 593 / 450; 40 x 262400 36.9 / 66.9, as 64 ranges leave it few workgroups).
+// Rows of two super-blocks are one launch of q4k_gemv16.hip (3000 x 512 at 8 / 24 tokens 8.5 / 8.7, this 9.4 /
+// 9.8; of one super-block 8.4 / 8.8, this 7.9 / 8.6).
 bool q6k_mid_takes(int N, int K, int M) {
   if (K > kF16Row) return M > 16 && M <= 32 && N >= 512 && K <= 4 * kF16Row;
+  if (K == 512 && M <= 32) return false;
   return M >= 2 && mid_takes(N, K, M, 1 << 24);
 }
 

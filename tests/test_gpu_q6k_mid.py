@@ -36,7 +36,8 @@ def tol(P):
 @pytest.mark.parametrize("out,in_,P", [(9, 256, 2), (127, 256, 16), (129, 512, 17), (260, 768, 32),
                                        (257, 1024, 33), (3584, 3584, 4), (300, 18944, 12),
                                        (3100, 24832, 3), (3000, 4096, 64), (2600, 2560, 50),
-                                       (640, 1792, 65), (1100, 5376, 128)])
+                                       (640, 1792, 65), (1100, 5376, 128), (127, 768, 16),
+                                       (129, 768, 17), (129, 512, 9), (130, 512, 32)])
 def test_shapes(hip, out, in_, P):
     print(f"[case] q6k mid out={out} in={in_} P={P}", flush=True)
     raw = weights(out, in_, seed=out + in_)
