@@ -10,7 +10,7 @@ namespace fhip {
 // Activation operands for 32-wide K slices. For slice s, lane group g (0..3) and operand row
 // rho = 2t + h (token t, h = 0 hi / 1 lo):
 //   A[(s * 4 + g) * 2M + rho] = 8 f16 values split_h(X[t][32 s + 8 g + perm8(j)] / e), j = 0..7
-//   E[(s >> 3) * M * 8 + t * 8 + (s & 7)] = {sum over the slice of (hi + lo), e}   (f32 pair)
+//   E[(s >> 3) * M * 8 + t * 8 + (s & 7)] = e
 // with e = 2^k chosen per (slice, token) so that the slice's largest magnitude lands in
 // [2^13, 2^14): any finite f32 activation block, however large or small, becomes f16 values
 // without overflow and with 11-bit relative precision down to 2^-28 of the block maximum, and
@@ -20,13 +20,13 @@ namespace fhip {
 // The same layout is used in LDS (staged by the matmul workgroup itself) and in global memory
 // (written by q8_xprep_kernel when the operands do not fit in LDS).
 
-// One (slice, token) task: 32 activations -> 8 operand rows + {sum, e}.
+// One (slice, token) task: 32 activations -> 8 operand rows + e.
 template <int M>
 __device__ __forceinline__ void split_slice(const float *__restrict__ x, bool valid, int sl,
                                             int t, uint4 *__restrict__ A,
-                                            float2 *__restrict__ E) {
+                                            float *__restrict__ E) {
   constexpr int R2 = 2 * M;
-  float sum = 0.f, e = 0.f;
+  float e = 0.f;
   if (valid) {
     float4 v[8];
 #pragma unroll
@@ -51,10 +51,8 @@ __device__ __forceinline__ void split_slice(const float *__restrict__ x, bool va
       for (int j = 0; j < 8; ++j) {
         const float xv = finite ? ldexpf(el[perm8(j)], -k) : 0.f;
         const _Float16 h = (_Float16)xv;
-        const _Float16 l = (_Float16)(xv - (float)h);
         hi[j] = h;
-        lo[j] = l;
-        sum += (float)h + (float)l;
+        lo[j] = (_Float16)(xv - (float)h);
       }
       A[(sl * 4 + g) * R2 + 2 * t] = __builtin_bit_cast(uint4, hi);
       A[(sl * 4 + g) * R2 + 2 * t + 1] = __builtin_bit_cast(uint4, lo);
@@ -66,7 +64,7 @@ __device__ __forceinline__ void split_slice(const float *__restrict__ x, bool va
       A[(sl * 4 + g) * R2 + 2 * t + 1] = make_uint4(0, 0, 0, 0);
     }
   }
-  E[(sl >> 3) * M * 8 + t * 8 + (sl & 7)] = make_float2(sum, e);
+  E[(sl >> 3) * M * 8 + t * 8 + (sl & 7)] = e;
 }
 
 // Stage slices [s0, s0 + ns) of M tokens (global slices >= ns_valid are zero) into A/E, whose
@@ -75,7 +73,7 @@ __device__ __forceinline__ void split_slice(const float *__restrict__ x, bool va
 template <int M>
 __device__ __forceinline__ void stage_x(const float *__restrict__ X, int K, int s0, int ns,
                                         int ns_valid, uint4 *__restrict__ A,
-                                        float2 *__restrict__ E, int lane, int nlanes) {
+                                        float *__restrict__ E, int lane, int nlanes) {
   for (int task = lane; task < ns * M; task += nlanes) {
     const int t = task / ns, sl = task - t * ns;
     const bool valid = s0 + sl < ns_valid;
@@ -86,7 +84,7 @@ __device__ __forceinline__ void stage_x(const float *__restrict__ X, int K, int 
 // Bytes of the operand layout for `ns` slices (E padded to whole groups of 8 slices).
 __host__ __device__ inline size_t xop_a_bytes(int M, int ns) { return (size_t)ns * 4 * 2 * M * 16; }
 __host__ __device__ inline size_t xop_bytes(int M, int ns) {
-  return xop_a_bytes(M, ns) + (size_t)((ns + 7) / 8) * M * 8 * 8;
+  return xop_a_bytes(M, ns) + (size_t)((ns + 7) / 8) * M * 8 * 4;
 }
 
 // Workgroup split-K: the KW waves of a 16-row tile each hold a partial over their own K part.

@@ -74,11 +74,10 @@ def test_17_to_32_tokens(hip, fmt, out, in_, P):
 @pytest.mark.parametrize("out,in_,P", [(33, 1 << 21, 40), (33, (1 << 21) + 32, 2), (17, (1 << 21) + 64, 16),
                                        (50, (1 << 21) + 32, 35)])
 def test_q8_0(hip, out, in_, P):
-    """The longest row of the GEMM, and rows past it: the GEMV in slices of sixteen tokens. Its per-row
-    rounding (products of 1152 + code less 1152 times the sum) is a few 2^-20: 2e-5."""
+    """The longest row of the GEMM, and rows past it: the GEMV in slices of sixteen tokens."""
     print(f"[case] long rows q8_0 out={out} in={in_} P={P}", flush=True)
     nb = in_ // 32
-    check("q8_0", out, in_, P, sorted({0, 1, P - 1}), [0, 1, 7, 8, nb // 2, nb // 2 + 1, nb - 2, nb - 1], 2e-5)
+    check("q8_0", out, in_, P, sorted({0, 1, P - 1}), [0, 1, 7, 8, nb // 2, nb // 2 + 1, nb - 2, nb - 1], 1e-5)
 
 
 @pytest.mark.parametrize("in_,P", [(1 << 20, 130), ((1 << 19) + 32, 300), (65536, 1000)])

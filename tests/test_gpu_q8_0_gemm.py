@@ -54,7 +54,7 @@ def test_range_lengths(hip, out, in_, P):
                                        (40000, 1056, 8), (40000, 1056, 9)])
 def test_few_tokens_of_a_large_matrix(hip, out, in_, P):
     """Three to eight tokens of 32 M weights and more, on either side of the rule that picks the GEMV or the
-    GEMM, and nine. The GEMV's products of 1152 + code less 1152 times the sum round to a few 2^-20: 2e-5."""
+    GEMM, and nine."""
     print(f"[case] q8_0 few tokens out={out} in={in_} P={P}", flush=True)
     rows = spread_rows(out)
     few = synth.q8_0_weights(len(rows), in_, seed=out + in_)
@@ -62,7 +62,7 @@ def test_few_tokens_of_a_large_matrix(hip, out, in_, P):
     raw[rows] = few.reshape(len(rows), -1)
     X = synth.activations(P, in_, P)
     Y = q8_0_matmul(raw.reshape(-1), out, in_, X, P)
-    assert rel_err_rows(Y[:, rows], exact(few, len(rows), in_, X)) <= 2e-5
+    assert rel_err_rows(Y[:, rows], exact(few, len(rows), in_, X)) <= 1e-5
     Y[:, rows] = 0
     assert not Y.any()
 
@@ -121,11 +121,21 @@ def test_small_blocks_beside_large_ones(hip, out, in_, P):
 
 @pytest.mark.parametrize("out,in_,P", [(200, 2048, 8), (33, 1056, 16), (3584, 3584, 3)])
 def test_gemv_global_operands_forced(hip, monkeypatch, out, in_, P):
-    """FAK_HIP_GEMV_GLOBALX=1: the GEMV with its operands in global memory, up to 16 tokens. Products of
-    1152 + code less 1152 times the sum: a few 2^-20."""
+    """FAK_HIP_GEMV_GLOBALX=1: the GEMV with its operands in global memory, up to 16 tokens."""
     print(f"[case] q8_0 gemv global operands out={out} in={in_} P={P}", flush=True)
     raw = synth.q8_0_weights(out, in_, seed=out + in_)
     X = synth.activations(P, in_, P)
     with knobs(monkeypatch, FAK_HIP_GEMV_GLOBALX=1):
         Y = q8_0_matmul(raw, out, in_, X, P)
-    assert rel_err_rows(Y, exact(raw, out, in_, X)) <= 2e-5
+    assert rel_err_rows(Y, exact(raw, out, in_, X)) <= 1e-5
+
+
+@pytest.mark.parametrize("out,in_,P", [(1536, 576, 1), (3584, 3584, 1), (300, 20000, 1), (2048, 2048, 8), (512, 1056, 16)])
+def test_gemv_error(hip, out, in_, P):
+    """The GEMV's operands are the codes themselves and 22 bits of the activations: 2-norm error against 64
+    bits a few 2^-24 (with 1152 + code, less 1152 times the block's sum, it was 1.5e-6 to 2e-6)."""
+    print(f"[case] q8_0 gemv error out={out} in={in_} P={P}", flush=True)
+    raw = synth.q8_0_weights(out, in_, seed=out + in_)
+    X = synth.activations(P, in_, P)
+    ref = exact(raw, out, in_, X)
+    assert np.linalg.norm(q8_0_matmul(raw, out, in_, X, P) - ref) <= 4e-7 * np.linalg.norm(ref)
