@@ -444,7 +444,7 @@ namespace {
 constexpr int kF16Row = 262144;  // rows longer than this take hi and lo operands up to 32 tokens
 constexpr int kMidRanges = 64;  // what sum_ranges reads at once
 // Operands (at most 36 MB, by mid_takes) and partial results together stay well inside the 64 MiB of the
-// no-allocation entry, whatever the shape.
+// no-allocation entry, whatever the shape. (Longer rows come from Q6_K only, which has no such entry.)
 constexpr size_t kMidScratch = (size_t)48 << 20;
 
 struct MidPlan {
@@ -477,7 +477,7 @@ MidPlan plan_mid(int fmt, int N, int K, int M, int TT, int NW) {
   const int fit = NW == 8 ? 1 : 2;  // workgroups per CU
   p.xb = (size_t)TT * p.MTG * nblk * kSbUnits * 1024;
   for (int sk = 1; sk <= nblk && sk <= kMidRanges; ++sk) {
-    if (sk > 1 && fmt == 0 && p.xb + (size_t)sk * M * N * 4 > kMidScratch) break;
+    if (sk > 1 && K <= kF16Row && p.xb + (size_t)sk * M * N * 4 > kMidScratch) break;
     const long long wgs = (long long)p.tasks * sk;
     const float pace = fit == 1 ? m.wide : wgs <= cus ? m.one : m.two;
     const float rounds = wgs <= cus ? 1.f : (float)((wgs + fit * cus - 1) / (fit * cus));
